@@ -419,7 +419,7 @@ def bench_rayquery(args):
     log(f"rayquery: closest {closest_ms:.3f} ms, any {any_ms:.3f} ms per launch, wall {wall:.3f}s, hit {hits / n:.4f}")
     algo_bytes = RQ_BYTES_PER_QUERY * n
     achieved = algo_bytes / (closest_ms * 1e-3) / 1e9
-    kernel = "traceRefillKernel" if launch["closest"]["form"] == rayquery.Mesh.REFILL else "traceBatchKernel"
+    kernel = "traceKernel"
     result = {
         "metric": "spectral paths/s at fixed rel. RMSE vs fp64 ref; adjoint grads/s; HBM GB/s",
         "value": 2 * n * args.steps / wall,

@@ -2,13 +2,17 @@
 // Stands in for MeshShape::intersect over many rays (src/owe/scene/mesh.cpp:73-97) and the float
 // kernels' any-hit occludedMesh (src/owe/backends/gpu/shaders/geometry.slang:577-615).
 //
-// Two launch forms. One lane per ray (traceBatchKernel), 128 lanes per block: a wave lives until its
-// longest ray ends. Lane refill (traceRefillKernel): a persistent grid whose waves each own a
-// contiguous range of rays; a lane whose ray ends waits until `refill` lanes of its wave are idle,
-// then the idle lanes take the next rays of the range together, so the wave keeps most of its lanes
-// busy instead of waiting on its slowest ray. Both forms walk each ray identically and return the
-// same hits bit for bit. The traversal stack lives in LDS with the capacity the build proved
-// sufficient (bvh4.hpp), chosen from a few compiled sizes.
+// One kernel (traceKernel) of persistent waves, each owning a contiguous range of rays: a lane whose
+// ray has ended waits until `refill` lanes of its wave are idle; then those write their results and
+// take the next rays of the range together. The form of one lane per ray is the same kernel with 64
+// rays to a wave. Per step a wave either visits a node or tests a triangle, in all the lanes that are
+// at one (traverse.hpp): a ray meets a leaf in one node of eight, so testing the leaves of a node where
+// it is visited, as the transport kernels' traverseBvh4 does, ran the triangle test with 1 to 5 lanes
+// of 64. Bound by the bytes beyond L2 (85 M lines of 128 bytes for 8,388,608 closest queries on
+// 1,048,820 triangles, 90 MB of nodes and triangles against 4 MiB of L2 per XCD), no longer by VALU
+// issue: 4.02 → 2.01 ms closest and 3.05 → 1.51 ms any hit; 0.48 → 0.29 and 0.35 → 0.19 ms for 1,000,003
+// rays on 100,820 triangles; 4,096 rays on 20,480 triangles, bound by the longest ray's chain of
+// loads, stay at 0.033 and go from 0.028 to 0.025 ms.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -37,155 +41,83 @@ namespace {
 
 constexpr int kQueryBlock = 128;
 
-template <int kCap, bool kAny>
-__global__ __launch_bounds__(kQueryBlock) void traceBatchKernel(const WideNode* __restrict__ nodes,
-                                                                const TriRecord* __restrict__ tris,
-                                                                const float4* __restrict__ rays, uint64_t n,
-                                                                uint32_t* __restrict__ primOut,
-                                                                float* __restrict__ tOut) {
-    __shared__ uint32_t stack[kCap * kQueryBlock];
-    const uint64_t i = uint64_t(blockIdx.x) * kQueryBlock + threadIdx.x;
-    if (i >= n) return;  // no barrier follows: lanes past the end simply leave
-    const float4 r0 = rays[2 * i], r1 = rays[2 * i + 1];
-    const RayHit h = traverseBvh4<kAny>(nodes, tris, mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), r0.w, r1.w, ~0u,
-                                        stack + threadIdx.x, kQueryBlock);
-    if (h.slot == kEmptyChild) {
-        primOut[i] = 0xFFFFFFFFu;
-        tOut[i] = __builtin_inff();
-    } else {
-        primOut[i] = tris[h.slot].prim;
-        tOut[i] = h.t;
-    }
-}
-
-// Result staging of the refill form. A wave takes its rays in increasing order, so they end in nearly
-// that order, but a lane's store of its own result touches a cache line that no neighbour has filled
-// yet. Each wave therefore holds kStageSlots LDS slots of 64 results: group g of its range (rays
-// start + 64g … start + 64g + 63) is staged in slot g % kStageSlots when that slot is free as the
-// wave first takes a ray of g, and leaves as one coalesced 64-lane store per output array once all
-// of its rays have ended. A group whose slot is still held writes its results directly, so a slow
-// ray never holds back the refill.
-constexpr uint32_t kStageSlots = 4;
-constexpr uint32_t kNoGroup = 0xFFFFFFFFu;
-
-// Persistent lanes with refill: wave w owns rays [w·per, min(n, (w + 1)·per)). Every branch that
-// decides a refill or a flush is wave-uniform (ballots, the range and the slots' owners); no barrier
-// is used, so waves run independently and each exits once its range is drained and its lanes are
-// idle, by which time every staged group has been flushed.
-template <int kCap, bool kAny>
-__global__ __launch_bounds__(kQueryBlock) void traceRefillKernel(const WideNode* __restrict__ nodes,
-                                                                 const TriRecord* __restrict__ tris,
-                                                                 const float4* __restrict__ rays, uint64_t n,
-                                                                 uint64_t per, uint32_t refill,
-                                                                 uint32_t* __restrict__ primOut,
-                                                                 float* __restrict__ tOut) {
-    __shared__ uint32_t stack[kCap * kQueryBlock];
-    __shared__ uint2 staged[kQueryBlock / 64][kStageSlots][64];
+// Wave w owns rays [w·per, min(n, (w + 1)·per)). Every branch that decides a refill or the step's kind is
+// wave-uniform (ballots and the range); no barrier is used, so waves run independently and each exits
+// once its range is drained and its lanes are idle. Results are written at a refill, many lanes
+// at once; lanes end out of order, so the lines fill in a few partial writes that L2 gathers.
+// The triangle step runs when the lanes at a leaf are half as many as those at a node, or when none is at
+// a node: of thresholds from a quarter to one and a half, and of fixed counts from 1 to 32, this one
+// was the fastest closest query (2.01 ms; 8 lanes fixed 2.4, 24 lanes fixed 2.3) and none was faster for any hit.
+template <bool kAny>
+__global__ __launch_bounds__(kQueryBlock) void traceKernel(const WideNode* __restrict__ nodes,
+                                                           const TriRecord* __restrict__ tris,
+                                                           const float4* __restrict__ rays, uint64_t n, uint64_t per,
+                                                           uint32_t refill, uint32_t* __restrict__ primOut,
+                                                           float* __restrict__ tOut) {
+    __shared__ uint32_t stack[kWalkLds * kQueryBlock];
+    uint32_t mem[kWalkStack - kWalkLds];
+    const WalkStack st{stack + threadIdx.x, mem};
     const uint32_t lane = threadIdx.x & 63u;
-    uint2(*stage)[64] = staged[threadIdx.x >> 6];
-    const uint64_t wave = (uint64_t(blockIdx.x) * kQueryBlock + threadIdx.x) >> 6;
-    const uint64_t start = wave * per;
-    uint64_t next = start;
+    const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kQueryBlock / 64) + (threadIdx.x >> 6));
+    uint64_t next = wave * per;
     const uint64_t end = next < n ? (n - next < per ? n : next + per) : next;
-    uint32_t owner[kStageSlots], held[kStageSlots];
-#pragma unroll
-    for (uint32_t j = 0; j < kStageSlots; ++j) owner[j] = kNoGroup, held[j] = 0;
-    uint32_t opened = 0;  // groups of the range whose slot has been decided
-    TravState s;
-    uint64_t ray = 0;
-    bool active = false;
+    constexpr uint64_t kNoRay = ~0ull;
+    uint64_t ray = kNoRay;  // the ray of this lane whose result is not written yet
+    Walk s;
+    s.hit.slot = s.cur = kEmptyChild;
     for (;;) {
-        const uint64_t idle = __ballot(!active);
-        const uint32_t nIdle = uint32_t(__popcll(idle));
-        if (next < end && (nIdle >= refill || nIdle == 64u)) {
-            const uint32_t rank = uint32_t(__popcll(idle & ((1ull << lane) - 1ull)));
-            if (!active && next + rank < end) {
+        const bool idle = s.cur == kEmptyChild;
+        const uint64_t idleMask = __ballot(idle);
+        const uint32_t nIdle = uint32_t(__popcll(idleMask));
+        if (nIdle == 64u || (next < end && nIdle >= refill)) {
+            if (idle && ray != kNoRay) {
+                const bool miss = s.hit.slot == kEmptyChild;
+                primOut[ray] = miss ? 0xFFFFFFFFu : tris[s.hit.slot].prim;
+                tOut[ray] = miss ? __builtin_inff() : s.hit.t;
+                ray = kNoRay;
+            }
+            if (next >= end) break;
+            const uint32_t rank = uint32_t(__popcll(idleMask & ((1ull << lane) - 1ull)));
+            if (idle && next + rank < end) {
                 ray = next + rank;
                 const float4 r0 = rays[2 * ray], r1 = rays[2 * ray + 1];
-                beginBvh4(s, mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), r0.w, r1.w);
-                active = true;
+                walkBegin(s, mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), r0.w, r1.w);
             }
             next = end - next > nIdle ? next + nIdle : end;
-            // The taken rays (at least one: refill ≥ 1) span at most two new groups; each takes its
-            // slot if the slot is free.
-            const uint32_t last = uint32_t((next - 1 - start) >> 6);
-            for (; opened <= last; ++opened) {
-#pragma unroll
-                for (uint32_t j = 0; j < kStageSlots; ++j)
-                    if (opened % kStageSlots == j && owner[j] == kNoGroup) owner[j] = opened, held[j] = 0;
-            }
         }
-        if (__ballot(active) == 0) break;
-        bool done = false;
-        uint32_t prim = 0;
-        float t = 0.0f;
-        if (active && stepBvh4<kAny>(s, nodes, tris, stack + threadIdx.x, kQueryBlock)) {
-            prim = s.hit.slot == kEmptyChild ? 0xFFFFFFFFu : tris[s.hit.slot].prim;
-            t = s.hit.slot == kEmptyChild ? __builtin_inff() : s.hit.t;
-            active = false;
-            done = true;
-        }
-        if (__ballot(done) == 0) continue;
-        const uint32_t group = uint32_t((ray - start) >> 6), slot = group % kStageSlots;
-        bool staging = false;
-#pragma unroll
-        for (uint32_t j = 0; j < kStageSlots; ++j) staging |= slot == j && owner[j] == group;
-        if (done) {
-            if (staging) {
-                stage[slot][(ray - start) & 63u] = make_uint2(prim, __float_as_uint(t));
-            } else {
-                primOut[ray] = prim;
-                tOut[ray] = t;
-            }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kStageSlots; ++j) {
-            held[j] += uint32_t(__popcll(__ballot(done && staging && slot == j)));
-            if (owner[j] == kNoGroup) continue;
-            const uint64_t base = start + 64ull * owner[j];
-            const uint32_t size = end - base < 64u ? uint32_t(end - base) : 64u;
-            if (held[j] != size) continue;
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            if (lane < size) {
-                const uint2 e = stage[j][lane];
-                primOut[base + lane] = e.x;
-                tOut[base + lane] = __uint_as_float(e.y);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            owner[j] = kNoGroup;
-            held[j] = 0;
+        const bool active = s.cur != kEmptyChild;
+        const bool atLeaf = active && (s.cur & kLeafBit) != 0;
+        const uint32_t leaves = uint32_t(__popcll(__ballot(atLeaf)));
+        const uint32_t inner = uint32_t(__popcll(__ballot(active && !atLeaf)));
+        if (2 * leaves >= inner) {
+            if (atLeaf) walkTriangle<kAny>(s, tris, st, kQueryBlock);
+        } else {
+            if (active && !atLeaf) walkNode(s, nodes, st, kQueryBlock);
         }
     }
 }
 
-template <int kCap>
 void launchTrace(int mode, const owe_hip_mesh* m, const float* rays, uint64_t n, uint32_t* prim, float* t,
                  hipStream_t s) {
-    const float4* r4 = reinterpret_cast<const float4*>(rays);
     const int q = mode == OWE_HIP_QUERY_ANY ? 1 : 0;
+    constexpr uint64_t kWaves = kQueryBlock / 64;
+    uint64_t blocks, per = 64;
+    uint32_t refill = 64;
     if (m->form[q] == OWE_HIP_TRACE_REFILL) {
-        const uint64_t blocks = uint64_t(m->cus) * uint64_t(m->blocksPerCu[q]);
-        const uint64_t waves = blocks * (kQueryBlock / 64);
-        const uint64_t per = (n + waves - 1) / waves;
-        const dim3 grid{unsigned(blocks)}, block{unsigned(kQueryBlock)};
-        if (mode == OWE_HIP_QUERY_ANY)
-            hipLaunchKernelGGL((traceRefillKernel<kCap, true>), grid, block, 0, s, m->nodes, m->tris, r4, n, per,
-                               uint32_t(m->refill[q]), prim, t);
-        else
-            hipLaunchKernelGGL((traceRefillKernel<kCap, false>), grid, block, 0, s, m->nodes, m->tris, r4, n, per,
-                               uint32_t(m->refill[q]), prim, t);
-        OWE_HIP_CHECK(hipGetLastError());
-        return;
+        blocks = uint64_t(m->cus) * uint64_t(m->blocksPerCu[q]);
+        per = (n + blocks * kWaves - 1) / (blocks * kWaves);
+        refill = uint32_t(m->refill[q]);
+    } else {
+        blocks = (n + kQueryBlock - 1) / kQueryBlock;
+        if (blocks > 0x7FFFFFFFull) fail(OWE_HIP_ERR_INVALID, "batch too large for one launch");
     }
-    const uint64_t blocks = (n + kQueryBlock - 1) / kQueryBlock;
-    if (blocks > 0x7FFFFFFFull) fail(OWE_HIP_ERR_INVALID, "batch too large for one launch");
     const dim3 grid{unsigned(blocks)}, block{unsigned(kQueryBlock)};
-    if (mode == OWE_HIP_QUERY_ANY)
-        hipLaunchKernelGGL((traceBatchKernel<kCap, true>), grid, block, 0, s, m->nodes, m->tris,
-                           reinterpret_cast<const float4*>(rays), n, prim, t);
-    else
-        hipLaunchKernelGGL((traceBatchKernel<kCap, false>), grid, block, 0, s, m->nodes, m->tris,
-                           reinterpret_cast<const float4*>(rays), n, prim, t);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, m->nodes, m->tris, reinterpret_cast<const float4*>(rays), n, per,
+                           refill, prim, t);
+    };
+    if (mode == OWE_HIP_QUERY_ANY) go(traceKernel<true>);
+    else go(traceKernel<false>);
     OWE_HIP_CHECK(hipGetLastError());
 }
 
@@ -295,11 +227,7 @@ int owe_hip_trace_batch(owe_hip_mesh* m, int mode, const float* rays, uint64_t n
         }
         OWE_HIP_CHECK(hipSetDevice(m->device));
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        const uint32_t cap = m->stats.stack_bound;
-        if (cap <= 16) launchTrace<16>(mode, m, rays, n, prim, t, s);
-        else if (cap <= 32) launchTrace<32>(mode, m, rays, n, prim, t, s);
-        else if (cap <= 48) launchTrace<48>(mode, m, rays, n, prim, t, s);
-        else launchTrace<64>(mode, m, rays, n, prim, t, s);
+        launchTrace(mode, m, rays, n, prim, t, s);
     });
 }
 

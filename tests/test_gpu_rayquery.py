@@ -162,3 +162,37 @@ def test_refill_form_returns_the_per_lane_forms_hits_bit_for_bit(cuda, n):
     assert mesh.launch(_lib.QUERY_ANY)["form"] == 0 and mesh.launch(_lib.QUERY_CLOSEST)["form"] == 1
     assert [run(mesh, closest), run(mesh, any_rays, _lib.QUERY_ANY)][1][0].tolist() == ref[1][0].tolist()
     print(f"n {n}: refill form identical over 4 shapes", flush=True)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 4097])
+def test_stacks_deeper_than_the_lds_part(cuda, oracle, n):
+    """Large overlapping triangles: rays hold more entries than a lane's LDS part of the stack, at
+    wave and block remainders; closest hit as the oracle's, any hit wherever the oracle has one."""
+    rng = np.random.default_rng(11)
+    c = rng.uniform(-1, 1, size=(60000, 1, 3))
+    pos = (c + rng.uniform(-1.5, 1.5, (60000, 3, 3))).reshape(-1, 3).astype(np.float32)
+    tri = np.arange(len(pos), dtype=np.uint32).reshape(-1, 3)
+    rays, _ = workloads.query_rays(n, seed=13)
+    rays[: n // 2, 7] = rng.uniform(0.2, 1.5, n // 2)  # many rays end before their first crossing
+    mesh = rayquery.Mesh(pos, tri)
+    assert mesh.stats().stack_bound > 20
+    op, ot = oracle.mesh(pos, tri).closest(rays)
+    for form in (rayquery.Mesh.REFILL, rayquery.Mesh.PER_LANE):
+        mesh.set_launch(form)
+        gp, gt = run(mesh, rays)
+        res = classify(pos, tri, rays, gp, gt, op, ot)
+        assert len(res["bad"]) == 0 and res["ties"] + res["grazing"] <= 1e-4 * n + 2
+        # t = (v0 - o)·N / d·N with N = e1 × e2: each factor of 3-vectors rounds to a few ulps of the
+        # product of its lengths, so |Δt| is within 16 ulps of |v0 - o| |e1| |e2| / |d·N| (slivers
+        # and grazing rays, where d·N is small, are what makes it exceed 1e-5 t here).
+        hit = (gp != MISS) & (gp == op)
+        v = pos[tri[gp[hit]]].astype(np.float64)
+        o, d = rays[hit, 0:3].astype(np.float64), rays[hit, 4:7].astype(np.float64)
+        e1, e2 = v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]
+        size = (np.linalg.norm(v[:, 0] - o, axis=1) * np.linalg.norm(e1, axis=1) * np.linalg.norm(e2, axis=1))
+        bound = 16 * 2.0**-23 * size / np.abs((d * np.cross(e1, e2)).sum(1))
+        assert (np.abs(gt[hit] - ot[hit]) <= bound).all()
+        ap, at = run(mesh, rays, _lib.QUERY_ANY)
+        tie = np.abs(ot - rays[:, 7]) <= 1e-5 * rays[:, 7]
+        assert (((ap != MISS) == np.isfinite(ot)) | tie).all()
+        assert (at[ap != MISS] < rays[ap != MISS, 7]).all()
