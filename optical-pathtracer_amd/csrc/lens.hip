@@ -1,15 +1,14 @@
 // Batched lens analysis: owe_hip_lens_batch_* of include/owe_hip_lens.h.
 //
 // Work is a flat list of items — (lens, wavelength, block of `raysPerItem` rays) — drained by a
-// persistent grid: each wave takes the next item with one atomic, its lanes trace the block's rays
-// through the lens surface after surface, reduce the spot's sums across the wave in double and add
+// persistent grid: each block takes the next few items with one atomic, its threads trace an item's rays
+// through the lens surface after surface, reduce the spot's sums across each wave in double and add
 // them to the (lens, wavelength) totals with one atomic per sum; arrived rays also land on the lens's
 // through-focus stack of detector grids as 64-bit fixed-point weights, so the irradiance is
-// independent of order. The grid adds gather first in a per-wave hash table in LDS (bin → sum),
-// which a wave flushes to HBM when its items move to another lens: a spot covers few bins, so most
-// of a lens's rays meet a bin already in the table and HBM sees about one atomic per bin touched
-// instead of one per ray. Lenses of very different ray counts (4k to 1M) share the launch without
-// tails of idle blocks.
+// independent of order. The grid adds gather first in the block's hash table in LDS (bin → sum),
+// flushed to HBM when its items move to another lens: most of a lens's rays meet a bin already in
+// the table and HBM sees about one atomic per bin touched instead of one per ray. Lenses of very
+// different ray counts (4k to 1M) share the launch without tails of idle blocks.
 //
 // Ray–surface roots follow SagSurface (src/owe/scene/geometry.cpp:115-166,
 // src/owe/core/shared/surfaces.hpp:13-94) in float32 with the reference's float tolerances; each
@@ -40,10 +39,13 @@ namespace {
 
 constexpr int kLensBlock = 256;
 constexpr double kHistScale = 4294967296.0;  // 2^32 units of weight per unit
-// The per-wave bin table: open addressing over kHashSlots (bin, sum) pairs, at most kHashProbes
-// probes before an add goes straight to HBM.
-constexpr int kHashSlots = 512;
+// A block's bin table: open addressing over kHashSlots (bin, sum) pairs, at most kHashProbes probes
+// before an add goes straight to HBM. An aberrated lens's five planes touch 1,000 bins and more: a table
+// of 512 slots to each wave was crowded and sent most adds to HBM (the kernel waited on them for
+// two thirds of its time), while 48 KiB to a block leave the three blocks to a compute unit that its registers allow.
+constexpr int kHashSlots = 4096;
 constexpr int kHashProbes = 8;
+constexpr uint32_t kPlaneGroup = 8;
 constexpr uint32_t kHashEmpty = 0xFFFFFFFFu;
 // The steepness |c|·r_max above which a quadric root is polished in float64.
 constexpr double kSteepPolish = 0.5;
@@ -52,6 +54,8 @@ constexpr double kSteepPolish = 0.5;
 // position along the fixed chart, and whether it reflects.
 struct DSurf : DSag {
     float z;
+    float gap;  // signed distance along the chart to the next row's vertex
+    double gapD;
     int32_t reflect;
 };
 
@@ -67,18 +71,23 @@ struct DLensInfo {
     uint32_t itemsPerLambda;
     uint32_t rings;           // 0: Fibonacci lattice; r: hexapolar rings
     double rEP, zEP, zStart;  // entrance pupil (sampling radius 0.999 rEP) and launch plane
+    double yStart;            // the launch plane's offset in y of a pupil point's ray
     float detX, detY, detZ, detHalf;  // detector grid centre, plane, half size (0: no grid)
+    float detScale;           // pixels per metre of the grid
     float detStep;            // through-focus plane spacing along z
+    float refB;               // afocal: a slope near the rays' (the paraxial apparent angle's) and its angle
+    double refA;
     int32_t afocal;           // spot sums of angles (afocalSpot) instead of (A, B) at an image
     int32_t mirrors;          // reflecting rows: their vertex planes obstruct
+    uint64_t mirrorMask;      // which of the first 64 rows reflect
 };
 
 struct LensArgs {
     const DSurf* surf;
     const DLensInfo* lens;
-    const float* nAfter;      // [surface × nλ]: index after each surface
-    const float* nAmbient;    // [lens × nλ]
+    const float* eta;         // [surface × nλ]: index before over index after each surface
     uint32_t nLenses, nLambda, raysPerItem, pixels, planes;
+    uint32_t chunk;           // consecutive items a block takes at a time
     uint64_t totalItems;
     double dirY, dirZ;        // collimated field direction (0, sin θ, cos θ)
     unsigned long long* next;
@@ -91,6 +100,36 @@ struct LensArgs {
     double* grads;
     int32_t sums;             // a gradient pass also adds the moments and histogram
 };
+
+// Quotients and roots of normal values to about an ulp: the hardware's estimate and one Newton step (two
+// for a double quotient's reciprocal), where the correctly rounded forms take 11 to 20 instructions and
+// their last half ulp is far below the rounding of the coordinates they lead to.
+__device__ __forceinline__ float quick(float num, float den) {
+    const float r = __builtin_amdgcn_rcpf(den);
+    return num * (r * (2.0f - den * r));
+}
+__device__ __forceinline__ double quick(double num, double den) {
+    double r = __builtin_amdgcn_rcp(den);
+    r = r * (2.0 - den * r);
+    const double v = num * (r * (2.0 - den * r));
+    return v + r * (num - v * den);
+}
+__device__ __forceinline__ float invSqrt(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    return y * (1.5f - 0.5f * x * y * y);
+}
+__device__ __forceinline__ float quickSqrt(float x) {  // 0 for x ≤ 0
+    x = fmaxf(x, 1e-30f);
+    const float y = __builtin_amdgcn_rsqf(x), v = x * y;
+    return v + 0.5f * y * (x - v * v);
+}
+__device__ __forceinline__ double quickSqrt(double x) {
+    x = fmax(x, 1e-280);
+    double y = __builtin_amdgcn_rsq(x);
+    y = y * (1.5 - 0.5 * x * y * y);
+    const double v = x * y;
+    return v + 0.5 * y * (x - v * v);
+}
 
 // Pupil point i of n on the entrance pupil of radius rEP, in double: a Fibonacci lattice over the
 // disc of radius 0.999 rEP, or with rings > 0 spotAt's hexapolar pattern (analysis.cpp:124-131) —
@@ -113,7 +152,7 @@ __device__ __forceinline__ void pupilPoint(uint64_t i, uint64_t n, uint32_t ring
     }
     // The lattice in float: the golden-ratio fraction of i from 64-bit fixed point (exact for any
     // i), the radius and angle to float rounding.
-    const float rr = 0.999f * float(rEP) * sqrtf((float(i) + 0.5f) / float(n));
+    const float rr = 0.999f * float(rEP) * quickSqrt(quick(float(i) + 0.5f, float(n)));
     const float f = float(uint32_t((i * 0x9E3779B97F4A7C15ull) >> 40)) * 0x1p-24f;
     float sa, ca;
     sincospif(2.0f * f, &sa, &ca);
@@ -121,18 +160,24 @@ __device__ __forceinline__ void pupilPoint(uint64_t i, uint64_t n, uint32_t ring
     y = double(rr * sa);
 }
 
-// Whether the ray o + s d, s in (0, sEnd) (sEnd < 0: unbounded), crosses the vertex-plane annulus
-// hole ≤ r ≤ semi-diameter of a mirror of the lens other than surfaces `from` and `to`.
+// Whether the ray from o along d, up to z = zEnd, crosses the vertex-plane annulus hole ≤ r ≤
+// semi-diameter of a mirror of the lens other than rows `from` and `to`. Only mirrors' rows are read:
+// those of the first 64 rows from the lens's mask, any later ones by looking.
+__device__ __forceinline__ bool obstructs(const DSurf& m, f3 o, f3 d, float zEnd) {
+    if (!(m.z > fminf(o.z, zEnd) && m.z < fmaxf(o.z, zEnd))) return false;
+    const float s = (m.z - o.z) / d.z;
+    const float x = o.x + d.x * s, y = o.y + d.y * s, r2 = x * x + y * y;
+    return r2 >= m.rMin2 && r2 <= m.rMax2;
+}
 __device__ __forceinline__ bool obstructed(const LensArgs& a, const DLensInfo& L, f3 o, f3 d, float zEnd, uint32_t from,
                                            uint32_t to) {
-    for (uint32_t j = 0; j < L.count; ++j) {
-        const DSurf& m = a.surf[L.first + j];
-        if (!m.reflect || j == from || j == to || d.z == 0.0f) continue;
-        if (!(m.z > fminf(o.z, zEnd) && m.z < fmaxf(o.z, zEnd))) continue;
-        const float s = (m.z - o.z) / d.z;
-        const float x = o.x + d.x * s, y = o.y + d.y * s, r2 = x * x + y * y;
-        if (r2 >= m.rMin2 && r2 <= m.rMax2) return true;
+    if (d.z == 0.0f) return false;
+    for (uint64_t left = L.mirrorMask; left != 0; left &= left - 1) {
+        const uint32_t j = uint32_t(__ffsll((long long)left)) - 1;
+        if (j != from && j != to && obstructs(a.surf[L.first + j], o, d, zEnd)) return true;
     }
+    for (uint32_t j = 64; j < L.count; ++j)
+        if (j != from && j != to && a.surf[L.first + j].reflect && obstructs(a.surf[L.first + j], o, d, zEnd)) return true;
     return false;
 }
 
@@ -141,20 +186,61 @@ struct RayGrad {
     float o[3][kGroup], d[3][kGroup];
 };
 
+// A conic or flat row met from o (z from its vertex) along unit d: from the vertex plane z = 0, where the
+// quadric c (x² + y² + (1 + k) z²) = 2 z has the constant term c (x² + y²) and its root on the vertex's sheet
+// is the small one C / w, which loses no digits; T: float, or double on rows with polish64. N is the
+// unnormalised normal (−c x, −c y, 1 − (1 + k) c z). The other root w / A is no crossing of this row where
+// there is none (A = 0), where it lies on the conic's other sheet, or behind o. kHit: the small root is the
+// first crossing; kMiss: the ray does not cross the row; kOther: neither is shown (the ray's z-part does
+// not dominate at the vertex plane, or the other root may be a crossing that comes first or alone), and
+// sagHit decides.
+enum { kMiss, kHit, kOther };
+template <class T>
+__device__ __forceinline__ int conicHit(const DSurf& sf, T c, T ck, T ox, T oy, T oz, T dx, T dy, T dz, float& th, f3& q,
+                                        f3& N) {
+    const T tv = quick(-oz, dz);
+    const T x0 = ox + dx * tv, y0 = oy + dy * tv;
+    const T A = c * (dx * dx + dy * dy) + ck * dz * dz;
+    const T B = c * (x0 * dx + y0 * dy) - dz;
+    const T C = c * (x0 * x0 + y0 * y0);
+    const T disc = B * B - A * C;
+    if (!(B * dz < T(0))) return kOther;
+    if (disc < T(0)) return kMiss;
+    const T w = -(B + copysign(quickSqrt(disc), B));
+    const T t2 = quick(C, w), t = tv + t2;
+    const T x = x0 + dx * t2, y = y0 + dy * t2, z = dz * t2;
+    q = mk3(float(x), float(y), float(z));
+    N = mk3(float(-c * x), float(-c * y), float(T(1) - ck * z));
+    th = float(t);
+    const bool first = A * dz < T(0);  // the other root comes before this one
+    const bool none = A == T(0) || ck * dz * w * A > T(1.001) * A * A || (first && (tv * A + w) * w > T(1e-3) * w * w);
+    const bool fits = t > T(0) && sagAccept(sf, q) && N.z >= -1e-6f;
+    if (fits) return first && !none ? kOther : kHit;
+    return none ? kMiss : kOther;
+}
+
 // One ray i of lens L at wavelength w: true when every surface takes it — a refracting row refracts
 // it, a mirror reflects it — no mirror body stops it and it leaves along +z; p, d after the last
 // surface. With kGrad the derivatives of p and d ride along (launch rays held fixed): at each
 // surface the implicit function theorem on F = sag(r²) − z gives the root's derivative
 // dt = −(∇F·(do + t dd) + dz_v + F_θ)/F_t, the hit point dp = do + t dd + dt d, the normal's through
 // dN of N = (−2g x, −2g y, 1) with g = d sag / d r², and the refracted or reflected direction's by
-// the chain rule of its formula.
+// the chain rule of its formula. A parameter of a later row has no derivative yet and is skipped
+// (uniformly: 37 of 48 row-parameter pairs are left of the Gregorian's eight).
+// Bound by VALU issue. The vertex-plane root, one cosine for Fresnel and Snell, one division for both
+// Fresnel amplitudes and the second-order renormalisation take about a third of the instructions of
+// the general quadric with its second solve (refineRoot) and separate formulas, and lie closer to the
+// 64-bit trace: 64 achromats (84 M rays, five planes) 5.87 → 3.14 ms; 32 Gregorians with eight
+// derivatives 2.54 → 1.38 ms.
 template <bool kGrad>
-__device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo& L, uint32_t li, uint32_t w, uint64_t i,
-                                             f3& p, f3& d, float& T, RayGrad& G) {
-    double x, y;
-    pupilPoint(i, L.rays, L.rings, L.rEP, x, y);
-    const double s = (L.zStart - L.zEP) / a.dirZ;
-    f3 o = mk3(float(x), float(y + a.dirY * s), float(L.zEP + a.dirZ * s));
+__device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo& L, uint32_t w, uint64_t i, f3& p, f3& d,
+                                             float& T, RayGrad& G) {
+    double px, py;
+    pupilPoint(i, L.rays, L.rings, L.rEP, px, py);
+    // o: z from the vertex of the row to be met, oz the same in double for rows with polish64 (a gap's
+    // rounding to float defocuses a high magnification by 10⁻⁴ of its spot).
+    f3 o = mk3(float(px), float(py + L.yStart), float(L.zStart));
+    double oz = L.zStart;
     d = mk3(0.0f, float(a.dirY), float(a.dirZ));
     T = 1.0f;
     if (kGrad) {
@@ -163,35 +249,51 @@ __device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo&
 #pragma unroll
             for (int k = 0; k < kGroup; ++k) G.o[c][k] = G.d[c][k] = 0.0f;
     }
-    float nPrev = a.nAmbient[li * a.nLambda + w];
     for (uint32_t k = 0; k < L.count; ++k) {
         const DSurf& sf = a.surf[L.first + k];
         f3 q, n;
         float th;
-        if (!sagHit(sf, mk3(o.x, o.y, o.z - sf.z), d, 0.0f, __builtin_inff(), false, th, q)) return false;
-        if (L.mirrors && obstructed(a, L, o, d, q.z + sf.z, k == 0 ? L.count : k - 1, k)) return false;
-        n = sagNormalF(sf, q);
+        int met = kOther;
+        if (sf.nA == 0) {
+            f3 N;
+            met = sf.polish64 ? conicHit<double>(sf, sf.c, sf.ck, o.x, o.y, oz, d.x, d.y, d.z, th, q, N)
+                              : conicHit<float>(sf, sf.cf, sf.ckf, o.x, o.y, o.z, d.x, d.y, d.z, th, q, N);
+            if (met == kMiss) return false;
+            n = N * invSqrt(dot3(N, N));
+        }
+        if (met == kOther) {
+            if (!sagHit(sf, o, d, 0.0f, __builtin_inff(), false, th, q)) return false;
+            n = sagNormalF(sf, q);
+        }
+        if (L.mirrors && obstructed(a, L, mk3(o.x, o.y, o.z + sf.z), d, q.z + sf.z, k == 0 ? L.count : k - 1, k)) return false;
+        const float dn = dot3(d, n);
+        const float eta = sf.reflect ? 1.0f : a.eta[(L.first + k) * a.nLambda + w];
+        float ct = 0.0f;
         f3 wv;
-        float eta = 1.0f;
         if (sf.reflect) {
-            wv = d - n * (2.0f * dot3(d, n));
+            wv = d - n * (2.0f * dn);
         } else {
-            const float nNext = a.nAfter[(L.first + k) * a.nLambda + w];
-            const float R = fresnelDielectric(fabsf(dot3(d, n)), nNext / nPrev);
-            if (!refractDir(d, n, nPrev, nNext, wv)) return false;
-            T *= 1.0f - R;
-            eta = nPrev / nNext;
-            nPrev = nNext;
+            // Snell and Fresnel share the cosines: r_s = (η c_i − c_t)/(η c_i + c_t), r_p = (c_i − η c_t)/(c_i + η c_t).
+            const float ci = fminf(fabsf(dn), 1.0f), k2 = 1.0f - eta * eta * (1.0f - ci * ci);
+            if (k2 < 0.0f) return false;
+            ct = quickSqrt(k2);
+            const float ps = eta * ci + ct, pp = ci + eta * ct;
+            const float inv = quick(1.0f, ps * pp);
+            const float rs = (eta * ci - ct) * pp * inv, rp = (ci - eta * ct) * ps * inv;
+            T *= 1.0f - 0.5f * (rs * rs + rp * rp);
+            const f3 u = d * eta + n * (copysignf(ct, dn) - eta * dn);
+            wv = u * (1.5f - 0.5f * dot3(u, u));  // |u| = 1 to rounding
         }
         if (kGrad) {
             // The surface's partials at the local hit point q.
             const float r2 = q.x * q.x + q.y * q.y, c = sf.cf, kk = sf.kf;
-            const float S = sqrtf(fmaxf(1e-30f, 1.0f - (1.0f + kk) * c * c * r2));
-            float g = c / (2.0f * S), gr = c * (1.0f + kk) * c * c / (4.0f * S * S * S);
-            const float Fc = r2 * ((1.0f + S) + (1.0f + kk) * r2 * c * c / S) / ((1.0f + S) * (1.0f + S));
-            const float Fk = c * c * c * r2 * r2 / (2.0f * S * (1.0f + S) * (1.0f + S));
-            const float gc = 1.0f / (2.0f * S) + (1.0f + kk) * c * c * r2 / (2.0f * S * S * S);
-            const float gk = c * c * c * r2 / (4.0f * S * S * S);
+            const float S2 = fmaxf(1e-30f, 1.0f - (1.0f + kk) * c * c * r2), iS = invSqrt(S2), S = S2 * iS;
+            const float i1 = quick(1.0f, 1.0f + S), iS3 = iS * iS * iS, c3 = c * c * c;
+            float g = 0.5f * c * iS, gr = 0.25f * (1.0f + kk) * c3 * iS3;
+            const float Fc = r2 * ((1.0f + S) + (1.0f + kk) * r2 * c * c * iS) * i1 * i1;
+            const float Fk = 0.5f * c3 * r2 * r2 * iS * i1 * i1;
+            const float gc = 0.5f * (iS + (1.0f + kk) * c * c * r2 * iS3);
+            const float gk = 0.25f * c3 * r2 * iS3;
             float FA[4], gA[4], rj = 1.0f;  // rj = r2^j
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -204,56 +306,42 @@ __device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo&
                 rj *= r2;
             }
             const f3 gradF = mk3(2.0f * g * q.x, 2.0f * g * q.y, -1.0f);
-            const float Ft = dot3(gradF, d);
+            const float iFt = quick(1.0f, dot3(gradF, d));
             const f3 N = mk3(-2.0f * g * q.x, -2.0f * g * q.y, 1.0f);
-            const float invN = rsqrtf(dot3(N, N));
-            const float sig = dot3(d, n) < 0.0f ? 1.0f : -1.0f;  // the refraction's facing normal
-            f3 W = wv;
-            float invW = 1.0f, ci = 0.0f, sq = 0.0f;
-            if (!sf.reflect) {
-                const f3 nn = n * sig;
-                ci = -dot3(d, nn);
-                sq = sqrtf(fmaxf(0.0f, 1.0f - eta * eta * (1.0f - ci * ci)));
-                W = d * eta + nn * (eta * ci - sq);
-                invW = rsqrtf(dot3(W, W));
-            }
+            const float invN = invSqrt(dot3(N, N));
+            const float sig = dn < 0.0f ? 1.0f : -1.0f;  // the refraction's facing normal
+            const float ci = fabsf(dn), kd = ct > 1e-15f ? quick(eta * eta * ci, ct) : 0.0f;  // d c_t = kd · d c_i
 #pragma unroll
             for (int kp = 0; kp < kGroup; ++kp) {
                 const uint32_t pi = a.paramBase + uint32_t(kp);
-                float dc = 0.0f, dk = 0.0f, dA[4] = {0.0f, 0.0f, 0.0f, 0.0f}, dzv = 0.0f;
-                if (pi < a.nParams) {
-                    const uint32_t ps = uint32_t(a.paramSurface[pi]);
-                    const int pf = a.paramField[pi];
-                    if (ps == k) {
-                        if (pf == OWE_LENS_PARAM_CURVATURE) dc = 1.0f;
-                        else if (pf == OWE_LENS_PARAM_CONIC) dk = 1.0f;
-                        else if (pf >= OWE_LENS_PARAM_A4) dA[pf - OWE_LENS_PARAM_A4] = 1.0f;
-                    }
-                    if (pf == OWE_LENS_PARAM_THICKNESS && ps < k) dzv = 1.0f;
+                if (pi >= a.nParams || uint32_t(a.paramSurface[pi]) > k) continue;
+                const uint32_t ps = uint32_t(a.paramSurface[pi]);
+                const int pf = a.paramField[pi];
+                const float dzv = pf == OWE_LENS_PARAM_THICKNESS && ps < k ? 1.0f : 0.0f;
+                float Fth = 0.0f, gth = 0.0f;
+                if (ps == k) {
+                    if (pf == OWE_LENS_PARAM_CURVATURE) Fth = Fc, gth = gc;
+                    if (pf == OWE_LENS_PARAM_CONIC) Fth = Fk, gth = gk;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (pf == OWE_LENS_PARAM_A4 + j) Fth = FA[j], gth = gA[j];
                 }
                 const f3 dO = mk3(G.o[0][kp], G.o[1][kp], G.o[2][kp]), dD = mk3(G.d[0][kp], G.d[1][kp], G.d[2][kp]);
-                float Fth = Fc * dc + Fk * dk, gth = gc * dc + gk * dk;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    Fth += FA[j] * dA[j];
-                    gth += gA[j] * dA[j];
-                }
                 const f3 dx = dO + dD * th;
-                const float dt = -(dot3(gradF, dx) + dzv + Fth) / Ft;
+                const float dt = -(dot3(gradF, dx) + dzv + Fth) * iFt;
                 const f3 dP = dx + d * dt;
                 // dN from dg = gr dr² + g_θ and the local point's move.
                 const float dg = gr * 2.0f * (q.x * dP.x + q.y * dP.y) + gth;
                 const f3 dN = mk3(-2.0f * (dg * q.x + g * dP.x), -2.0f * (dg * q.y + g * dP.y), 0.0f);
-                const f3 dn = (dN - n * dot3(n, dN)) * invN;
+                const f3 dnv = (dN - n * dot3(n, dN)) * invN;
                 f3 dW;
                 if (sf.reflect) {
-                    dW = dD - (n * (dot3(dD, n) + dot3(d, dn)) + dn * dot3(d, n)) * 2.0f;
+                    dW = dD - (n * (dot3(dD, n) + dot3(d, dnv)) + dnv * dn) * 2.0f;
                 } else {
-                    const f3 nn = n * sig, dnn = dn * sig;
+                    const f3 nn = n * sig, dnn = dnv * sig;
                     const float dci = -(dot3(dD, nn) + dot3(d, dnn));
-                    const float dsq = sq > 0.0f ? eta * eta * ci * dci / sq : 0.0f;
-                    const f3 dWu = dD * eta + nn * (eta * dci - dsq) + dnn * (eta * ci - sq);
-                    dW = (dWu - wv * dot3(wv, dWu)) * invW;
+                    // (No renormalisation: the refracted direction of unit vectors is one.)
+                    dW = dD * eta + nn * (dci * (eta - kd)) + dnn * (eta * ci - ct);
                 }
                 G.o[0][kp] = dP.x;
                 G.o[1][kp] = dP.y;
@@ -263,7 +351,9 @@ __device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo&
                 G.d[2][kp] = dW.z;
             }
         }
-        o = mk3(q.x, q.y, q.z + sf.z);
+        const bool last = k + 1 == L.count;
+        o = mk3(q.x, q.y, last ? q.z + sf.z : q.z - sf.gap);
+        oz = double(q.z) - sf.gapD;
         d = wv;
     }
     if (L.mirrors && obstructed(a, L, o, d, d.z > 0.0f ? __builtin_inff() : -__builtin_inff(), L.count - 1, L.count))
@@ -272,40 +362,59 @@ __device__ __forceinline__ bool traceLensRay(const LensArgs& a, const DLensInfo&
     return d.z > 0.0f;
 }
 
-__device__ __forceinline__ double waveSumD(double v) {
+// The sums over a wave of N values per lane (N a power of two up to 32): lanes exchange halves of what they
+// hold, so N + log2(64 / N) − 1 exchanges do what N separate sums take 6 N for. The sum of value j ends
+// in v[0] of the lanes whose top log2(N) bits are j.
+template <int N, int kHalf = N / 2>
+__device__ __forceinline__ void waveSums(double (&v)[N], uint32_t lane) {
+    if constexpr (kHalf >= 1) {
+        constexpr int off = 64 * kHalf / N;
+        const bool high = (lane & uint32_t(off)) != 0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
+        for (int j = 0; j < kHalf; ++j) {
+            const double give = high ? v[j] : v[j + kHalf], keep = high ? v[j + kHalf] : v[j];
+            v[j] = keep + __shfl_xor(give, off);
+        }
+        waveSums<N, kHalf / 2>(v, lane);
+    } else {
+#pragma unroll
+        for (int off = 32 / N; off >= 1; off /= 2) v[0] += __shfl_xor(v[0], off);
+    }
 }
 
-// A wave's bin table in LDS. Keys are bins of the lens the wave is on (plane · pixels² + row ·
+// The block's bin table in LDS. Keys are bins of the lens the block is on (plane · pixels² + row ·
 // pixels + column); a key is claimed by compare-and-swap, its sum grown by a 64-bit LDS add.
 struct BinTable {
     uint32_t* keys;
     unsigned long long* sums;
 };
 
-__device__ __forceinline__ void binAdd(BinTable t, unsigned long long* lensHist, uint32_t key, unsigned long long v) {
-    uint32_t slot = (key * 2654435761u) >> (32 - 9);
-    static_assert(kHashSlots == 512, "the slot hash takes 9 bits");
+__device__ __forceinline__ uint32_t binSlot(uint32_t key) {
+    static_assert(kHashSlots == 1 << 12, "the slot hash takes 12 bits");
+    return (key * 2654435761u) >> (32 - 12);
+}
+// held: what the key's slot was last seen to hold. A claimed slot never changes before the flush, so
+// a read (one for all lanes of a bin) finds most keys and only a first visitor swaps.
+__device__ __forceinline__ void binAdd(BinTable t, unsigned long long* lensHist, uint32_t key, uint32_t held,
+                                       unsigned long long v) {
+    uint32_t slot = binSlot(key);
 #pragma unroll 1
     for (int probe = 0; probe < kHashProbes; ++probe) {
-        const uint32_t old = atomicCAS(&t.keys[slot], kHashEmpty, key);
-        if (old == kHashEmpty || old == key) {
+        if (held == kHashEmpty) held = atomicCAS(&t.keys[slot], kHashEmpty, key);
+        if (held == kHashEmpty || held == key) {
             atomicAdd(&t.sums[slot], v);
             return;
         }
         slot = (slot + 1) & uint32_t(kHashSlots - 1);
+        held = t.keys[slot];
     }
     atomicAdd(lensHist + key, v);  // the table is crowded here: straight to HBM
 }
 
-// Adds every claimed bin of the table to the lens's grids and empties the table. Wave-wide: every
-// lane takes part, after every lane's adds (the fence keeps the compiler from moving LDS accesses
-// across it; one wave's LDS operations complete in order).
-__device__ __forceinline__ void binFlush(BinTable t, unsigned long long* lensHist, uint32_t lane) {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    for (uint32_t q = lane; q < uint32_t(kHashSlots); q += 64) {
+// Adds every claimed bin of the table to the lens's grids and empties the table. By the whole block,
+// between barriers.
+__device__ __forceinline__ void binFlush(BinTable t, unsigned long long* lensHist) {
+    for (uint32_t q = threadIdx.x; q < uint32_t(kHashSlots); q += kLensBlock) {
         const uint32_t key = t.keys[q];
         if (key != kHashEmpty) {
             atomicAdd(lensHist + key, t.sums[q]);
@@ -313,31 +422,42 @@ __device__ __forceinline__ void binFlush(BinTable t, unsigned long long* lensHis
             t.sums[q] = 0;
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
-// The persistent batch: a wave takes the next (lens, wavelength, block of rays) item, its lanes
-// trace the block, the spot sums (and with kGrad the derivative sums of the pass's parameters) are
-// reduced across the wave in double and added with one atomic each; grid adds go through the
-// wave's bin table, flushed when the wave's next item is another lens's and before it exits.
+// The persistent batch: a block takes the next `chunk` consecutive (lens, wavelength, block of rays)
+// items, its threads trace each item's rays, the spot sums (and with kGrad the derivative sums of the
+// pass's parameters) are reduced across each wave in double and added with one atomic each; grid
+// adds go through the block's bin table, flushed when an item is another lens's and before the block
+// exits. Chunks keep a block on one lens for most of its life, so few tables are flushed. Every
+// barrier is reached by the whole block: items and their lens are uniform across it.
 template <bool kGrad>
 __global__ __launch_bounds__(kLensBlock) void lensKernel(LensArgs a) {
-    __shared__ uint32_t tableKeys[kLensBlock / 64][kHashSlots];
-    __shared__ unsigned long long tableSums[kLensBlock / 64][kHashSlots];
+    __shared__ uint32_t tableKeys[kHashSlots];
+    __shared__ unsigned long long tableSums[kHashSlots];
+    __shared__ unsigned long long firstItem;
     const uint32_t lane = __lane_id();
     const bool sums = !kGrad || a.sums;
     const bool grids = sums && a.pixels > 0;
-    const BinTable table{tableKeys[threadIdx.x / 64], tableSums[threadIdx.x / 64]};
-    for (uint32_t q = lane; q < uint32_t(kHashSlots); q += 64) {
-        table.keys[q] = kHashEmpty;
-        table.sums[q] = 0;
-    }
+    const BinTable table{tableKeys, tableSums};
+    if (grids)
+        for (uint32_t q = threadIdx.x; q < uint32_t(kHashSlots); q += kLensBlock) {
+            table.keys[q] = kHashEmpty;
+            table.sums[q] = 0;
+        }
     const size_t lensBins = size_t(a.planes) * a.pixels * a.pixels;
     uint32_t tableLens = ~0u;  // the lens whose bins the table holds
+    uint64_t item = 0, lastItem = 0;
     for (;;) {
-        unsigned long long item = 0;
-        if (lane == 0) item = atomicAdd(a.next, 1ull);
-        item = __shfl(item, 0);
+        if (item == lastItem) {
+            __syncthreads();  // every thread has read the previous chunk's first item
+            if (threadIdx.x == 0) firstItem = atomicAdd(a.next, (unsigned long long)a.chunk);
+            __syncthreads();
+            item = firstItem;
+            // Uniform in scalar registers, so the lens's rows are read through the scalar unit.
+            item = uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(item)))) |
+                   uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(item >> 32)))) << 32;
+            lastItem = item + a.chunk;
+        }
         if (item >= a.totalItems) break;
         // The lens of this item: the last whose first item is ≤ item.
         uint32_t lo = 0, len = a.nLenses;
@@ -353,28 +473,36 @@ __global__ __launch_bounds__(kLensBlock) void lensKernel(LensArgs a) {
         const uint32_t li = lo - 1;
         const DLensInfo& L = a.lens[li];
         if (grids && li != tableLens) {
-            if (tableLens != ~0u) binFlush(table, a.hist + tableLens * lensBins, lane);
+            __syncthreads();  // the table is clear, or every add of the previous lens is in it
+            if (tableLens != ~0u) {
+                binFlush(table, a.hist + tableLens * lensBins);
+                __syncthreads();
+            }
             tableLens = li;
         }
         unsigned long long* lensHist = a.hist + size_t(li) * lensBins;
         const uint64_t local = item - L.itemBase;
+        ++item;
         const uint32_t w = uint32_t(local / L.itemsPerLambda);
         const uint64_t first = (local % L.itemsPerLambda) * a.raysPerItem;
-        double m[OWE_LENS_MOMENTS] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        double m[OWE_LENS_MOMENTS - 1] = {0, 0, 0, 0, 0, 0, 0, 0};  // all but the count of arrived rays
+        uint32_t arrived = 0;
         float gs[kGrad ? kGroup : 1][kGradSums] = {};
-        for (uint32_t k = lane; k < a.raysPerItem; k += 64) {
+        for (uint32_t k = threadIdx.x; k < a.raysPerItem; k += kLensBlock) {
             const uint64_t i = first + k;
             if (i >= L.rays) break;
             f3 p, d;
             float T;
             RayGrad G;
-            if (!traceLensRay<kGrad>(a, L, li, w, i, p, d, T, G)) continue;
+            if (!traceLensRay<kGrad>(a, L, w, i, p, d, T, G)) continue;
             // The ray's spot terms in float (B = d_xy / d_z, A at z = 0 or the angles), summed in
-            // double.
-            const float iz = 1.0f / d.z;
+            // double. An afocal spot's variance is 10⁻⁴ and less of its mean square, so its y angles
+            // are taken relative to the angle refA of a slope refB near them, where float keeps their digits:
+            // atan b = refA + atan((b − refB) / (1 + b refB)).
+            const float iz = quick(1.0f, d.z);
             const float bx = d.x * iz, by = d.y * iz;
             const float ax = L.afocal ? atanf(bx) : p.x - bx * p.z;
-            const float ay = L.afocal ? atanf(by) : p.y - by * p.z;
+            const float ay = L.afocal ? atanf((by - L.refB) / (1.0f + by * L.refB)) : p.y - by * p.z;
             if (kGrad) {
 #pragma unroll
                 for (int kp = 0; kp < kGroup; ++kp) {
@@ -398,52 +526,72 @@ __global__ __launch_bounds__(kLensBlock) void lensKernel(LensArgs a) {
                 }
             }
             if (!sums) continue;
-            m[0] += 1.0;
-            m[1] += double(ax);
-            m[2] += double(ay);
-            m[3] += double(bx);
-            m[4] += double(by);
-            m[5] += double(ax * ax + ay * ay);
-            m[6] += double(bx * bx + by * by);
-            m[7] += double(ax * bx + ay * by);
-            m[8] += double(T);
+            ++arrived;
+            m[0] += double(ax);
+            m[2] += double(bx);
+            m[3] += double(by);
+            if (L.afocal) {
+                const double y = L.refA + double(ay);
+                m[1] += y;
+                m[4] += double(ax) * double(ax) + y * y;
+                m[6] += double(ax) * double(bx) + y * double(by);
+            } else {
+                m[1] += double(ay);
+                m[4] += double(ax * ax + ay * ay);
+                m[6] += double(ax * bx + ay * by);
+            }
+            m[5] += double(bx * bx + by * by);
+            m[7] += double(T);
             if (grids && L.detHalf > 0.0f) {
                 const unsigned long long v = (unsigned long long)llrint(double(T) * kHistScale);
-                const float half = 0.5f * float(a.planes - 1);
-                for (uint32_t pl = 0; pl < a.planes; ++pl) {
-                    const float z = L.detZ + (float(pl) - half) * L.detStep;
-                    const float s = (z - p.z) * iz;
-                    const float gx = (p.x + d.x * s - L.detX) / L.detHalf, gy = (p.y + d.y * s - L.detY) / L.detHalf;
-                    const float fx = (gx + 1.0f) * 0.5f * float(a.pixels), fy = (1.0f - gy) * 0.5f * float(a.pixels);
-                    if (fx >= 0.0f && fy >= 0.0f && fx < float(a.pixels) && fy < float(a.pixels)) {
+                const float half = 0.5f * float(a.planes - 1), mid = 0.5f * float(a.pixels);
+                // Groups of planes: their table reads are in flight together.
+                for (uint32_t first = 0; first < a.planes; first += kPlaneGroup) {
+                    uint32_t key[kPlaneGroup], held[kPlaneGroup];
+#pragma unroll
+                    for (uint32_t g = 0; g < kPlaneGroup; ++g) {
+                        key[g] = held[g] = kHashEmpty;
+                        const uint32_t pl = first + g;
+                        if (pl >= a.planes) continue;
+                        const float s = L.detZ + (float(pl) - half) * L.detStep - p.z;
+                        const float fx = mid + (p.x + bx * s - L.detX) * L.detScale;
+                        const float fy = mid - (p.y + by * s - L.detY) * L.detScale;
+                        if (!(fx >= 0.0f && fy >= 0.0f && fx < float(a.pixels) && fy < float(a.pixels))) continue;
                         const uint32_t px = min(uint32_t(fx), a.pixels - 1), py = min(uint32_t(fy), a.pixels - 1);
-                        binAdd(table, lensHist, (pl * a.pixels + py) * a.pixels + px, v);
+                        key[g] = (pl * a.pixels + py) * a.pixels + px;
+                        held[g] = table.keys[binSlot(key[g])];
                     }
+#pragma unroll
+                    for (uint32_t g = 0; g < kPlaneGroup; ++g)
+                        if (key[g] != kHashEmpty) binAdd(table, lensHist, key[g], held[g], v);
                 }
             }
         }
         if (sums) {
+            static_assert(OWE_LENS_MOMENTS == 9, "the arrived count and eight sums");
             double* dst = a.moments + (size_t(li) * a.nLambda + w) * OWE_LENS_MOMENTS;
+            waveSums(m, lane);
 #pragma unroll
-            for (int q = 0; q < OWE_LENS_MOMENTS; ++q) {
-                const double v = waveSumD(m[q]);
-                if (lane == 0 && v != 0.0) atomicAdd(dst + q, v);
-            }
+            for (int off = 32; off > 0; off >>= 1) arrived += __shfl_xor(arrived, off);
+            if (lane == 0 && arrived) atomicAdd(dst, double(arrived));
+            if ((lane & 7u) == 0 && m[0] != 0.0) atomicAdd(dst + 1 + (lane >> 3), m[0]);
         }
         if (kGrad) {
-            double* dst = a.grads + (size_t(li) * a.nLambda + w) * (OWE_LENS_MAX_PARAMS * kGradSums);
+            static_assert(kGroup * kGradSums <= 32, "a pass's derivative sums reduce together");
+            double g[32] = {};
 #pragma unroll
-            for (int kp = 0; kp < kGroup; ++kp) {
-                if (a.paramBase + uint32_t(kp) >= a.nParams) continue;
+            for (int kp = 0; kp < kGroup; ++kp)
 #pragma unroll
-                for (int q = 0; q < kGradSums; ++q) {
-                    const double v = waveSumD(double(gs[kp][q]));
-                    if (lane == 0 && v != 0.0) atomicAdd(dst + (a.paramBase + kp) * kGradSums + q, v);
-                }
-            }
+                for (int q = 0; q < kGradSums; ++q) g[kp * kGradSums + q] = double(gs[kp][q]);
+            waveSums(g, lane);
+            const uint32_t j = lane >> 1;
+            if ((lane & 1u) == 0 && j < kGroup * kGradSums && a.paramBase + j / kGradSums < a.nParams && g[0] != 0.0)
+                atomicAdd(a.grads + (size_t(li) * a.nLambda + w) * (OWE_LENS_MAX_PARAMS * kGradSums) +
+                              a.paramBase * kGradSums + j, g[0]);
         }
     }
-    if (grids && tableLens != ~0u) binFlush(table, a.hist + tableLens * lensBins, lane);
+    __syncthreads();
+    if (grids && tableLens != ~0u) binFlush(table, a.hist + tableLens * lensBins);
 }
 
 __global__ void lensBegin(LensArgs a, size_t nMoments, size_t nHist, size_t nGrads) {
@@ -466,7 +614,7 @@ __global__ void lensProbe(LensArgs a, uint32_t li, uint32_t w, const uint64_t* i
     float T;
     RayGrad G;
     double* r = out + 7 * k;
-    if (traceLensRay<false>(a, a.lens[li], li, w, index[k], p, d, T, G)) {
+    if (traceLensRay<false>(a, a.lens[li], w, index[k], p, d, T, G)) {
         r[0] = p.x, r[1] = p.y, r[2] = p.z, r[3] = d.x, r[4] = d.y, r[5] = d.z, r[6] = T;
     } else {
         for (int q = 0; q < 6; ++q) r[q] = __builtin_nan("");
@@ -596,7 +744,7 @@ struct owe_hip_lens_batch {
     LensArgs args{};
     size_t nMoments = 0, nHist = 0, nGrads = 0;
     int computeUnits = 256;
-    int blocksPerCU = 4;
+    int blocksPerCU = 3;  // what registers and LDS hold
     hipEvent_t ev[2] = {nullptr, nullptr};
     double lastMs = 0;
     bool ran = false;
@@ -627,12 +775,28 @@ void layoutItems(owe_hip_lens_batch* b, uint32_t raysPerItem) {
     b->args.totalItems = base;
 }
 
+// Rays per item before any tuning: eight items to each resident block, as a small batch needs every
+// compute unit (256 rays, one to a thread) and a large one fewer reductions (4,096 rays).
+uint32_t defaultItem(const owe_hip_lens_batch* b) {
+    uint64_t rays = 0;
+    for (const DLensInfo& L : b->info) rays += L.rays * b->args.nLambda;
+    const uint64_t per = rays / (uint64_t(b->computeUnits) * uint64_t(b->blocksPerCU) * 8);
+    return uint32_t(std::clamp<uint64_t>((per + kLensBlock - 1) / kLensBlock * kLensBlock, kLensBlock, 4096));
+}
+
+// The chunk of items a block takes at a time: four chunks to a block of the grid, so blocks stay on a lens
+// and the last chunks still even out.
+uint32_t chunkOf(const owe_hip_lens_batch* b, unsigned blocks) {
+    return uint32_t(std::clamp<uint64_t>(b->args.totalItems / (4 * uint64_t(blocks)), 1, 1u << 20));
+}
+
 // One run: the plain kernel, or with parameters set one gradient pass per kGroup parameters (the
 // first also adding the spot sums and the histogram).
 double runOnce(owe_hip_lens_batch* b) {
     hipLaunchKernelGGL(lensBegin, dim3{1024}, dim3{256}, 0, b->stream, b->args, b->nMoments, b->nHist, b->nGrads);
     OWE_HIP_CHECK(hipEventRecord(b->ev[0], b->stream));
     const dim3 grid{unsigned(std::max(1, b->computeUnits * b->blocksPerCU))};
+    b->args.chunk = chunkOf(b, grid.x);
     if (b->args.nParams == 0) {
         hipLaunchKernelGGL(lensKernel<false>, grid, dim3{kLensBlock}, 0, b->stream, b->args);
     } else {
@@ -701,7 +865,7 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
         OWE_HIP_CHECK(hipEventCreate(&b->ev[1]));
         const uint32_t nw = uint32_t(s.n_wavelengths);
         std::vector<DSurf> ds;
-        std::vector<float> nAfter(size_t(n_surfaces) * nw, 1.0f), nAmb(size_t(n_lenses) * nw, 1.0f);
+        std::vector<float> eta(size_t(n_surfaces) * nw, 1.0f);
         std::vector<uint8_t> used(n_surfaces, 0);
         // Lenses whose every root is polished in float64: instruments with mirrors or afocal ones,
         // where metre-long paths and the angular magnification turn a float root's error along
@@ -721,19 +885,22 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
             const owe_lens_surface* rows = surfaces + L.first_surface;
             std::vector<double> nRef(L.surface_count);
             int mirrors = 0;
+            uint64_t mirrorMask = 0;
             for (uint32_t k = 0; k < L.surface_count; ++k) {
                 require(!used[L.first_surface + k], name + ": surfaces are shared with another lens");
                 used[L.first_surface + k] = 1;
                 if (rows[k].reflect) {
                     ++mirrors;
+                    if (k < 64) mirrorMask |= uint64_t(1) << k;
                     require(rows[k].medium == (k == 0 ? L.ambient : rows[k - 1].medium),
                             name + ": a mirror reflects into the medium it is met in");
                 }
                 nRef[k] = mediumIndexHost(media[rows[k].medium], s.reference_wavelength);
+                const owe_medium& before = media[k == 0 ? L.ambient : rows[k - 1].medium];
                 for (uint32_t w = 0; w < nw; ++w)
-                    nAfter[size_t(L.first_surface + k) * nw + w] = float(mediumIndexHost(media[rows[k].medium], s.wavelengths[w]));
+                    eta[size_t(L.first_surface + k) * nw + w] =
+                        float(mediumIndexHost(before, s.wavelengths[w]) / mediumIndexHost(media[rows[k].medium], s.wavelengths[w]));
             }
-            for (uint32_t w = 0; w < nw; ++w) nAmb[size_t(li) * nw + w] = float(mediumIndexHost(media[L.ambient], s.wavelengths[w]));
             const ParaxialOut px = paraxialHost(rows, L.surface_count, nRef, mediumIndexHost(media[L.ambient], s.reference_wavelength));
             owe_lens_result r{};
             r.launched = L.rays * nw;
@@ -753,6 +920,7 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
             I.rEP = px.epr;
             I.zEP = px.epz;
             I.zStart = -0.05 - 0.1 * px.length;
+            I.yStart = std::sin(f) * ((I.zStart - I.zEP) / std::cos(f));
             // The detector: the paraxial image plane at the reference wavelength, centred on the
             // chief ray's paraxial image height EFL·tan θ.
             I.detZ = float(px.lastZ + px.bfl);
@@ -762,9 +930,13 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
             I.detStep = float(s.focus_step > 0 ? s.focus_step : 1e-3 * std::fabs(px.efl));
             I.afocal = px.afocal ? 1 : 0;
             I.mirrors = mirrors;
+            I.mirrorMask = mirrorMask;
+            I.refB = px.afocal ? float(px.angMag * std::tan(f)) : 0.0f;
+            I.refA = std::atan(double(I.refB));
             if (px.afocal) {  // no image plane: no irradiance grid
                 I.detZ = I.detY = I.detHalf = I.detStep = 0.0f;
             }
+            I.detScale = I.detHalf > 0 ? float(0.5 * s.detector_pixels / double(I.detHalf)) : 0.0f;
             b->info.push_back(I);
             precise.push_back(mirrors > 0 || px.afocal);
         }
@@ -779,6 +951,8 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
                                                 r.reflect ? r.hole_radius : 0.0);
                 d.polish64 = precise[li] || std::fabs(r.curvature) * r.semi_diameter > kSteepPolish ? 1 : 0;
                 d.z = float(z);
+                d.gap = float(r.thickness);
+                d.gapD = r.thickness;
                 d.reflect = r.reflect ? 1 : 0;
                 ds[L.first_surface + k] = d;
                 z += r.thickness;
@@ -790,12 +964,9 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
         OWE_HIP_CHECK(hipMemcpy(dsurf, ds.data(), ds.size() * sizeof(DSurf), hipMemcpyHostToDevice));
         a.surf = dsurf;
         a.lens = lensAlloc<DLensInfo>(b, n_lenses);
-        float* na = lensAlloc<float>(b, nAfter.size());
-        OWE_HIP_CHECK(hipMemcpy(na, nAfter.data(), nAfter.size() * sizeof(float), hipMemcpyHostToDevice));
-        a.nAfter = na;
-        float* nb = lensAlloc<float>(b, nAmb.size());
-        OWE_HIP_CHECK(hipMemcpy(nb, nAmb.data(), nAmb.size() * sizeof(float), hipMemcpyHostToDevice));
-        a.nAmbient = nb;
+        float* de = lensAlloc<float>(b, eta.size());
+        OWE_HIP_CHECK(hipMemcpy(de, eta.data(), eta.size() * sizeof(float), hipMemcpyHostToDevice));
+        a.eta = de;
         a.nLenses = n_lenses;
         a.nLambda = nw;
         a.pixels = uint32_t(s.detector_pixels);
@@ -810,7 +981,7 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
         b->nGrads = 0;
         a.grads = lensAlloc<double>(b, size_t(n_lenses) * nw * OWE_LENS_MAX_PARAMS * kGradSums);
         a.nParams = 0;
-        layoutItems(b, 1024);
+        layoutItems(b, defaultItem(b));
         *out = b;
     });
     if (st != OWE_HIP_OK && b) {
@@ -883,7 +1054,8 @@ int owe_hip_lens_batch_gradients(owe_hip_lens_batch* b, double* grad) {
             const double n = m[0];
             for (size_t k = 0; k < np; ++k) {
                 double out = NAN;
-                const double* G = &g[k * kGradSums];  // ΣA'x, ΣA'y, ΣB'x, ΣB'y, ΣA·A', ΣB·B', Σ(A'·B + A·B')
+                // ΣA'x, ΣA'y, ΣB'x, ΣB'y, ΣA·A', ΣB·B', Σ(A'·B + A·B'); afocal: A relative to (0, refA).
+                const double* G = &g[k * kGradSums];
                 if (n >= 3) {
                     const double max = m[1] / n, may = m[2] / n, mbx = m[3] / n, mby = m[4] / n;
                     const double dmax = G[0] / n, dmay = G[1] / n, dmbx = G[2] / n, dmby = G[3] / n;
@@ -892,8 +1064,10 @@ int owe_hip_lens_batch_gradients(owe_hip_lens_batch* b, double* grad) {
                         const double cx = std::atan(mbx), cy = std::atan(mby);
                         const double dcx = dmbx / (1 + mbx * mbx), dcy = dmby / (1 + mby * mby);
                         const double v = m[5] / n - 2 * (cx * max + cy * may) + cx * cx + cy * cy;
-                        const double dv = 2 * G[4] / n - 2 * (dcx * max + dcy * may) - 2 * (cx * dmax + cy * dmay) +
-                                          2 * (cx * dcx + cy * dcy);
+                        // v' = 2 E[(A − c)·A'] − 2 c'·(E A − c).
+                        const double ref = b->info[li].refA;
+                        const double dv = 2 * (G[4] / n - cx * dmax + (ref - cy) * dmay) -
+                                          2 * (dcx * (max - cx) + dcy * (may - cy));
                         out = v > 0 ? dv / (2 * std::sqrt(v)) : 0.0;
                     } else {
                         // rms² at best focus = var_A − cov²/var_B (focusedSpot).

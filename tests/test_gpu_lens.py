@@ -196,3 +196,37 @@ def test_through_focus_stack_matches_the_oracle_bin_by_bin(cuda, oracle):
               f"{got.max(axis=(1, 2))}", flush=True)
         assert close.mean() > 0.995
         assert np.abs(got.sum() - want.sum()) <= 1e-4 * want.sum()
+
+
+@pytest.mark.parametrize("field", [0.5, 30.0, 55.0])
+def test_conic_roots_of_every_form_match_oracle(cuda, oracle, field):
+    """Rows of either curvature, shallow to hemispherical, flat, ellipsoids, paraboloids and hyperboloids,
+    met steeply and at the edge of their apertures: the row's first crossing, whichever root it is.
+    A coordinate here is at most 0.3 m, so it rounds to 3e-8 m at most and a direction to that over the
+    row's radius (1 cm and more); 99 % of the rays stay within three and ten times those, the others graze
+    a row or the critical angle, where refraction magnifies without bound."""
+    rng = np.random.default_rng(int(field) + 3)
+    lenses = []
+    for k in range(48):
+        rows = []
+        for j in range(1 + k % 3):
+            R = rng.uniform(12, 80) * rng.choice((-1, 1)) if rng.random() < 0.9 else math.inf
+            conic = rng.choice((0.0, -1.0, rng.uniform(-2, 1)))
+            sd = rng.uniform(0.1, 0.95) * min(abs(R), 60.0) / math.sqrt(max(1.0, 1 + conic))
+            glass = "air" if j == 2 or (j == 1 and k % 2) else ("N-BK7", "N-SF11")[j % 2]
+            rows.append(L.Surface(R, rng.uniform(1.0, 30.0), glass, sd, k=conic, stop=j == 0))
+        lenses.append(L.Prescription(rows, rays=2048))
+    b = L.LensBatch(lenses, L.c_settings(field_deg=field))
+    lo = LensOracle(oracle, lenses, field_deg=field)
+    idx = np.arange(2048, dtype=np.uint64)
+    total = flips = far = 0
+    for li in range(len(lenses)):
+        g, c = b.trace(li, 4, idx), lo.trace(li, L.FRAUNHOFER7[4], idx)
+        both = (g[:, 6] > 0) & (c[:, 6] > 0)
+        total += int(both.sum())
+        flips += int(((g[:, 6] > 0) != (c[:, 6] > 0)).sum())
+        far += int(((np.abs(g[both, :3] - c[both, :3]).max(1) > 1e-7) |
+                    (np.abs(g[both, 3:6] - c[both, 3:6]).max(1) > 3e-5)).sum())
+    b.close()
+    print(f"field {field}: {total} rays arrive on both, {flips} flips, {far} beyond the bound", flush=True)
+    assert total > 20 * 2048 and flips <= total // 1000 and far <= total // 100
