@@ -101,36 +101,6 @@ struct LensArgs {
     int32_t sums;             // a gradient pass also adds the moments and histogram
 };
 
-// Quotients and roots of normal values to about an ulp: the hardware's estimate and one Newton step (two
-// for a double quotient's reciprocal), where the correctly rounded forms take 11 to 20 instructions and
-// their last half ulp is far below the rounding of the coordinates they lead to.
-__device__ __forceinline__ float quick(float num, float den) {
-    const float r = __builtin_amdgcn_rcpf(den);
-    return num * (r * (2.0f - den * r));
-}
-__device__ __forceinline__ double quick(double num, double den) {
-    double r = __builtin_amdgcn_rcp(den);
-    r = r * (2.0 - den * r);
-    const double v = num * (r * (2.0 - den * r));
-    return v + r * (num - v * den);
-}
-__device__ __forceinline__ float invSqrt(float x) {
-    const float y = __builtin_amdgcn_rsqf(x);
-    return y * (1.5f - 0.5f * x * y * y);
-}
-__device__ __forceinline__ float quickSqrt(float x) {  // 0 for x ≤ 0
-    x = fmaxf(x, 1e-30f);
-    const float y = __builtin_amdgcn_rsqf(x), v = x * y;
-    return v + 0.5f * y * (x - v * v);
-}
-__device__ __forceinline__ double quickSqrt(double x) {
-    x = fmax(x, 1e-280);
-    double y = __builtin_amdgcn_rsq(x);
-    y = y * (1.5 - 0.5 * x * y * y);
-    const double v = x * y;
-    return v + 0.5 * y * (x - v * v);
-}
-
 // Pupil point i of n on the entrance pupil of radius rEP, in double: a Fibonacci lattice over the
 // disc of radius 0.999 rEP, or with rings > 0 spotAt's hexapolar pattern (analysis.cpp:124-131) —
 // point 0 the centre, ring k holding the 6k points after the 1 + 3k(k − 1) before it.
@@ -389,6 +359,13 @@ struct BinTable {
     unsigned long long* sums;
 };
 
+// An add to LDS in the block's scope: with atomicAdd the compiler folds it and the add to HBM of a
+// crowded table into one through a generic pointer, which is several times slower.
+template <class V>
+__device__ __forceinline__ void ldsAdd(V* p, V v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 __device__ __forceinline__ uint32_t binSlot(uint32_t key) {
     static_assert(kHashSlots == 1 << 12, "the slot hash takes 12 bits");
     return (key * 2654435761u) >> (32 - 12);
@@ -402,7 +379,7 @@ __device__ __forceinline__ void binAdd(BinTable t, unsigned long long* lensHist,
     for (int probe = 0; probe < kHashProbes; ++probe) {
         if (held == kHashEmpty) held = atomicCAS(&t.keys[slot], kHashEmpty, key);
         if (held == kHashEmpty || held == key) {
-            atomicAdd(&t.sums[slot], v);
+            ldsAdd(&t.sums[slot], v);
             return;
         }
         slot = (slot + 1) & uint32_t(kHashSlots - 1);

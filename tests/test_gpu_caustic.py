@@ -174,3 +174,44 @@ def test_adjoint_costs_at_most_three_forwards(cuda):
     print(f"forward {f:.3f} ms, adjoint {b:.3f} ms, ratio {b / f:.2f} (1,048,576 particles)", flush=True)
     assert b <= 3.0 * f
     c.close()
+
+
+@pytest.mark.parametrize("particles", [1, 255, 257, 5000, 1 << 18])
+def test_adjoint_of_wide_ranges_and_remainders(cuda, particles):
+    """The adjoint's block sums choose their own unit: a wall whose right half's ∂L/∂E is 10⁻¹² of the
+    left's (or 10⁻³⁵, where no unit suits) gives the right's nodes what the right half alone gives, and
+    an infinite pixel reaches its nodes and no others. Sums of up to a few hundred float adds in another order
+    differ by at most as many half ulps: 2e-5 in norm."""
+    import torch
+
+    s = C.caustic_settings(nodes=64, pixels=128, particles=particles)
+    c = C.Caustic(s)
+    h = torch.tensor(C.initial_heights(64, feature=16), device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    base = torch.randn((128, 128), device="cuda", generator=g)
+    right = torch.zeros_like(base)
+    right[:, 64:] = base[:, 64:]
+    left = base - right
+
+    def adjoint(ge):
+        out = torch.empty_like(h)
+        c.backward_into(h, ge.contiguous(), out, 0)
+        torch.cuda.synchronize()
+        return out
+
+    alone = adjoint(right).double()
+    assert torch.isfinite(alone).all()
+    inner = alone[:, 40:]  # nodes whose particles land well inside the right half
+    for scale in (1.0, 1e-12, 1e12):
+        both = adjoint(left / scale + right)[:, 40:].double()
+        assert (both - inner).norm() <= 2e-5 * inner.norm()
+    tiny = adjoint(right * 1e-35)[:, 40:].double() * 1e35
+    assert (tiny - inner).norm() <= 1e-3 * inner.norm()  # products down to 1e-38 lose digits as floats
+    assert (adjoint(torch.zeros_like(base)) == 0).all()
+    spoiled = right.clone()
+    spoiled[64, 32] = float("inf")
+    got = adjoint(spoiled)
+    assert torch.isfinite(got[:, 40:]).all() and (got[:, 40:].double() - inner).norm() <= 2e-5 * inner.norm()
+    if particles >= 5000:
+        assert not torch.isfinite(got[:, :40]).all()
+    c.close()
