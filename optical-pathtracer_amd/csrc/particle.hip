@@ -681,7 +681,8 @@ __global__ __launch_bounds__(kPBlock) void particleKernel(DScene sc, Settings se
 // ends. Particle ids come in chunks of `chunk` from one device counter (one atomic per wave per
 // refill). The bins are integers, so the image equals particleKernel's bit for bit.
 template <bool kContacts>
-__global__ __launch_bounds__(kPBlock) void particleRefillKernel(DScene sc, Settings set, ParticleBatch pb) {
+__global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene* __restrict__ scene, Settings set, ParticleBatch pb) {
+    const DScene& sc = *scene;
     __shared__ uint32_t stack[kRefillStack * kPBlock];
     PCtx c{sc, set, pb, stack + threadIdx.x};
     c.sum[0] = c.sum[1] = c.sum[2] = 0.0f;
@@ -896,7 +897,8 @@ __device__ __forceinline__ void vcmLightPath(PCtx& c, const VcmDev& v, uint32_t 
 // One thread per light subpath j of slot k's iteration (thread k·N + j): its own stream (seed, j,
 // iteration) and the wavelengths of its group, j mod G (vcm_light_kernel.slang).
 template <bool kContacts>
-__global__ __launch_bounds__(kPBlock, OWE_HIP_VCM_WAVES) void vcmLightKernel(DScene sc, Settings set, VcmDev v, ParticleBatch pb) {
+__global__ __launch_bounds__(kPBlock, OWE_HIP_VCM_WAVES) void vcmLightKernel(const DScene* __restrict__ scene, Settings set, VcmDev v, ParticleBatch pb) {
+    const DScene& sc = *scene;
     __shared__ uint32_t stack[kRefillStack * kPBlock];
     const uint32_t t = blockIdx.x * kPBlock + threadIdx.x;
     PCtx c{sc, set, pb, stack + threadIdx.x};
@@ -984,7 +986,7 @@ void launchParticles(const DScene& sc, const Settings& set, const ParticleBatch&
     OWE_HIP_CHECK(hipGetLastError());
 }
 
-void launchVcmLight(const DScene& sc, const Settings& set, const VcmDev& v, unsigned long long* lightFilm,
+void launchVcmLight(bool contacts, const DScene* sc, const Settings& set, const VcmDev& v, unsigned long long* lightFilm,
                     unsigned long long* stats, float invNWY, uint32_t count, hipStream_t stream) {
     if (count == 0) return;
     ParticleBatch pb{};
@@ -993,16 +995,16 @@ void launchVcmLight(const DScene& sc, const Settings& set, const VcmDev& v, unsi
     pb.stats = stats;
     pb.invNWY = invNWY;
     const dim3 grid{(count + kPBlock - 1) / kPBlock}, block{kPBlock};
-    if (sc.contacts) hipLaunchKernelGGL((vcmLightKernel<true>), grid, block, 0, stream, sc, set, v, pb);
+    if (contacts) hipLaunchKernelGGL((vcmLightKernel<true>), grid, block, 0, stream, sc, set, v, pb);
     else hipLaunchKernelGGL((vcmLightKernel<false>), grid, block, 0, stream, sc, set, v, pb);
     OWE_HIP_CHECK(hipGetLastError());
 }
 
-void launchParticlesRefill(const DScene& sc, const Settings& set, const ParticleBatch& b, uint32_t blocks,
+void launchParticlesRefill(bool contacts, const DScene* sc, const Settings& set, const ParticleBatch& b, uint32_t blocks,
                            hipStream_t stream) {
     if (b.total == 0) return;
     const dim3 grid{std::max(1u, blocks)}, block{kPBlock};
-    if (sc.contacts) hipLaunchKernelGGL((particleRefillKernel<true>), grid, block, 0, stream, sc, set, b);
+    if (contacts) hipLaunchKernelGGL((particleRefillKernel<true>), grid, block, 0, stream, sc, set, b);
     else hipLaunchKernelGGL((particleRefillKernel<false>), grid, block, 0, stream, sc, set, b);
     OWE_HIP_CHECK(hipGetLastError());
 }

@@ -1594,7 +1594,8 @@ __device__ __forceinline__ void vcmMerge(VcmCamera& c, const VcmVertex& x) {
 // One camera path of pixel `pixel` in slot k's iteration (thread k·pixels + pixel; traceCameraVcm,
 // vcm.slang:523-593); its contributions, every strategy but light tracing, go to the camera film.
 template <bool kContacts>
-__global__ __launch_bounds__(kBlock, OWE_HIP_VCM_WAVES) void vcmCameraKernel(DScene sc, Settings set, VcmDev vAll, unsigned long long* stats) {
+__global__ __launch_bounds__(kBlock, OWE_HIP_VCM_WAVES) void vcmCameraKernel(const DScene* __restrict__ scene, Settings set, VcmDev vAll, unsigned long long* stats) {
+    const DScene& sc = *scene;
     __shared__ uint32_t stack[48 * kBlock];
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     const DObserver& ob = sc.obs;
@@ -1807,6 +1808,7 @@ struct owe_hip_renderer {
     int device = 0;
     HostScene host;
     DScene dev{};
+    DScene* scene = nullptr;  // dev in device memory, for the particle and vcm kernels (particle.hpp)
     Settings set{};
     std::vector<void*> allocations;
     Paths P{};
@@ -2169,7 +2171,7 @@ void runParticles(owe_hip_renderer* r, uint64_t total, uint32_t pass, const uint
         b.regen = r->regen;
         OWE_HIP_CHECK(hipMemsetAsync(r->particleNext, 0, sizeof(unsigned long long), r->stream));
         timed(r, kShade, [&] {
-            launchParticlesRefill(r->dev, r->set, b, uint32_t(std::max(1, r->computeUnits * r->blocksPerCU)), r->stream);
+            launchParticlesRefill(r->dev.contacts != 0u, r->scene, r->set, b, uint32_t(std::max(1, r->computeUnits * r->blocksPerCU)), r->stream);
         });
     } else {
         // One thread per particle, in launches of at most `capacity` particles.
@@ -2248,7 +2250,7 @@ void runVcm(owe_hip_renderer* r, int iterations) {
         if (r->host.emittedPower > 0) {
             const uint32_t tiles = (paths + kScanTile - 1) / kScanTile;
             timed(r, kGenerate,
-                  [&] { launchVcmLight(r->dev, r->set, v, r->lightFilm, r->particleStats, r->invNWY, paths, r->stream); });
+                  [&] { launchVcmLight(r->dev.contacts != 0u, r->scene, r->set, v, r->lightFilm, r->particleStats, r->invNWY, paths, r->stream); });
             hipLaunchKernelGGL(vcmTileSumKernel, dim3{tiles}, dim3{kScanBlock}, 0, r->stream, v.pathCount, paths, v.tileSum);
             hipLaunchKernelGGL(vcmScanKernel, dim3{1}, dim3{kScanThreads}, 0, r->stream, v.tileSum, v.tileOffset, tiles);
             hipLaunchKernelGGL(vcmScanCompactKernel, dim3{tiles}, dim3{kScanBlock}, 0, r->stream, v, paths);
@@ -2261,10 +2263,10 @@ void runVcm(owe_hip_renderer* r, int iterations) {
         }
         timed(r, kShade, [&] {
             if (r->dev.contacts)
-                hipLaunchKernelGGL((vcmCameraKernel<true>), gridFor(S * pixels), dim3{kBlock}, 0, r->stream, r->dev, r->set,
+                hipLaunchKernelGGL((vcmCameraKernel<true>), gridFor(S * pixels), dim3{kBlock}, 0, r->stream, r->scene, r->set,
                                    v, r->particleStats);
             else
-                hipLaunchKernelGGL((vcmCameraKernel<false>), gridFor(S * pixels), dim3{kBlock}, 0, r->stream, r->dev, r->set,
+                hipLaunchKernelGGL((vcmCameraKernel<false>), gridFor(S * pixels), dim3{kBlock}, 0, r->stream, r->scene, r->set,
                                    v, r->particleStats);
         });
         OWE_HIP_CHECK(hipGetLastError());
@@ -2601,6 +2603,8 @@ int owe_hip_renderer_create(int device, const owe_scene* scene, const owe_render
             r->chunk = 4;
             r->regen = 32;
         }
+        r->scene = devAlloc<DScene>(r, 1);
+        OWE_HIP_CHECK(hipMemcpy(r->scene, &r->dev, sizeof r->dev, hipMemcpyHostToDevice));
         *out = r;
     });
     if (st != OWE_HIP_OK && r) {

@@ -182,7 +182,7 @@ __device__ __forceinline__ bool vcmEval(const DScene& sc, const Iface& it, uint3
 
 // Enqueues the light subpaths [0, count) of the slots' iterations (light tracing into the particle
 // film's bins, the staging slots filled) on `stream`; count = slots · N.
-void launchVcmLight(const DScene& sc, const Settings& set, const VcmDev& v, unsigned long long* lightFilm,
+void launchVcmLight(bool contacts, const DScene* sc, const Settings& set, const VcmDev& v, unsigned long long* lightFilm,
                     unsigned long long* stats, float invNWY, uint32_t count, hipStream_t stream);
 
 }  // namespace owehip
