@@ -678,7 +678,7 @@ __global__ __launch_bounds__(kPBlock) void particleKernel(DScene sc, Settings se
 // particle deposits the same splats. A lane whose particle has ended waits until `regen` lanes of
 // its wave are idle; then they start the next particles of their chunks together, so the wave runs
 // the emission code once for many lanes and stays full instead of idling until its longest walk
-// ends. Particle ids come in chunks of `chunk` from one device counter (one atomic per wave per
+// ends. Particle ids come in chunks of up to `chunk` (grainOf) from one device counter (one atomic per wave per
 // refill). The bins are integers, so the image equals particleKernel's bit for bit.
 template <bool kContacts>
 __global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene* __restrict__ scene, Settings set, ParticleBatch pb) {
@@ -702,11 +702,16 @@ __global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene*
         if (ask) {
             const int leader = __ffsll((long long)ask) - 1;
             unsigned long long base = 0;
-            if (int(lane) == leader) base = atomicAdd(pb.next, (unsigned long long)__popcll(ask) * pb.chunk);
+            uint32_t grain = 0;
+            if (int(lane) == leader) {
+                grain = grainOf(pb.total - end, pb.chunk, gridDim.x * kPBlock);
+                base = atomicAdd(pb.next, (unsigned long long)__popcll(ask) * grain);
+            }
             base = __shfl(base, leader);
+            grain = __shfl(grain, leader);
             if (needChunk) {
-                id = base + uint64_t(__popcll(ask & ((1ull << lane) - 1ull))) * pb.chunk;
-                end = id + pb.chunk < pb.total ? id + pb.chunk : pb.total;
+                id = base + uint64_t(__popcll(ask & ((1ull << lane) - 1ull))) * grain;
+                end = id + grain < pb.total ? id + grain : pb.total;
                 done = id >= pb.total;
             }
         }

@@ -847,8 +847,8 @@ __global__ void setCount(uint32_t* c, unsigned long long* segments, uint32_t cou
 // The batched persistent form of the same camera loop: a grid sized to the chip keeps one path per
 // lane in registers and advances it one segment per iteration (intersect, shade, shadow — the very
 // device functions of the wavefront kernels, so every path's float operations are the same); a lane
-// whose path ends splats it and takes the next path id from its chunk, or a new chunk of `chunk`
-// consecutive ids from a device counter (one atomic per wave per refill). Splats of consecutive
+// whose path ends splats it and takes the next path id from its chunk, or a new chunk of up to `chunk`
+// consecutive ids (grainOf) from a device counter (one atomic per wave per refill). Splats of consecutive
 // paths of one pixel accumulate in the lane and reach the film as one 64-bit atomic per channel.
 // The film is integer, so it equals the wavefront's bit for bit.
 struct Persist {
@@ -917,11 +917,16 @@ __device__ __forceinline__ uint32_t persistDrain(const DScene& sc, const Setting
         if (ask) {
             const int leader = __ffsll((long long)ask) - 1;
             unsigned long long base = 0;
-            if (int(lane) == leader) base = atomicAdd(a.next, (unsigned long long)__popcll(ask) * a.chunk);
+            uint32_t grain = 0;
+            if (int(lane) == leader) {
+                grain = grainOf(a.total - end, a.chunk, gridDim.x * kBlock);
+                base = atomicAdd(a.next, (unsigned long long)__popcll(ask) * grain);
+            }
             base = __shfl(base, leader);
+            grain = __shfl(grain, leader);
             if (needChunk) {
-                id = base + uint64_t(__popcll(ask & ((1ull << lane) - 1ull))) * a.chunk;
-                end = id + a.chunk < a.total ? id + a.chunk : a.total;
+                id = base + uint64_t(__popcll(ask & ((1ull << lane) - 1ull))) * grain;
+                end = id + grain < a.total ? id + grain : a.total;
                 done = id >= a.total;
             }
         }

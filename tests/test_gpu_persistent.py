@@ -108,3 +108,16 @@ def test_autotune_picks_a_shape_and_leaves_no_trace(cuda):
     assert w.autotune(16) > 0 and w.mode()["mode"] == render.Renderer.WAVEFRONT
     w.run_pass(16)
     assert np.array_equal(w.resolve(), ref)
+
+
+@pytest.mark.parametrize("width,height,spp,chunk,blocks", [(101, 67, 170, 1024, 1), (64, 64, 16, 1024, 8), (3, 1, 1, 4, 2)])
+def test_shrinking_chunks_trace_every_path_once(cuda, width, height, spp, chunk, blocks):
+    # Chunks from a quarter of a lane's share down to one id: more ids than lanes by an odd factor, about one
+    # id a lane, and fewer ids than one wave's lanes. The film and the statistics are integers: no tolerance.
+    sc = S.dispersion_prism_scene(width, height)
+    st = S.settings(seed=12, **PRISM)
+    a, sa = render_with(sc, st, spp, 2, False)
+    b, sb = render_with(sc, st, spp, 2, True, blocks_per_cu=blocks, chunk=chunk, refill=32)
+    assert sa["paths"] == 2 * width * height * spp
+    assert np.array_equal(a, b)
+    assert sa == sb
