@@ -249,6 +249,9 @@ __global__ __launch_bounds__(kBlock) void generateKernel(DScene sc, Settings set
                                                           uint32_t spp, uint32_t pass, const uint32_t* pixelList,
                                                           const uint32_t* sampleList) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    // Queue 0 holds `count` paths, queue 1 none; no segments, inconsistencies or leaks yet.
+    if (i < 4) P.count[i] = i == 0 ? count : 0u;
+    if (i == 0) *P.segments = 0;
     if (i >= count) return;
     uint64_t pixel, s;
     if (pixelList) {
@@ -606,6 +609,30 @@ __device__ __forceinline__ bool shadeOne(ShadeCtx& c, const uint4 hraw, uint32_t
     return true;
 }
 
+// A live path's state from its records (r1: its direction and weight); shPend is left as it is.
+__device__ __forceinline__ void loadPath(ShadeCtx& c, const Paths& P, uint32_t slot, uint64_t passInc, float4& r1) {
+    const float4 r0 = P.ray0[slot];
+    r1 = P.ray1[slot];
+    const uint4 info = P.info[slot];
+    const uint2 rs = P.rng[slot];
+    c.rng.state = uint64_t(rs.x) | (uint64_t(rs.y) << 32);
+    c.rng.inc = passInc;
+    c.flags = info.y >> 16;
+    c.depth = info.y & 0xFFFFu;
+    c.wl = loadWL(P.lam[slot], c.flags, c.set);
+    c.beta = P.beta[slot];
+    c.L = P.L[slot];
+    c.o = mk3(r0.x, r0.y, r0.z);
+    c.prevPdf = r0.w;
+    c.d = mk3(r1.x, r1.y, r1.z);
+    const float4 pp = P.prevP[slot];
+    c.prevP = mk3(pp.x, pp.y, pp.z);
+    c.pixel = info.x;
+    c.region = info.z;
+    c.departed = info.w;
+    c.face = P.face[slot];
+}
+
 __global__ __launch_bounds__(kBlock) void shadeKernel(DScene sc, Settings set, Paths P, int q, uint64_t passInc) {
     const uint32_t count = P.count[q];
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
@@ -613,26 +640,9 @@ __global__ __launch_bounds__(kBlock) void shadeKernel(DScene sc, Settings set, P
     uint32_t slot = 0;
     if (k < count) {
         slot = P.queue[q][k];
-        const float4 r0 = P.ray0[slot], r1 = P.ray1[slot];
-        const uint4 info = P.info[slot];
-        const uint2 rs = P.rng[slot];
         ShadeCtx c{sc, set};
-        c.rng.state = uint64_t(rs.x) | (uint64_t(rs.y) << 32);
-        c.rng.inc = passInc;
-        c.flags = info.y >> 16;
-        c.depth = info.y & 0xFFFFu;
-        c.wl = loadWL(P.lam[slot], c.flags, set);
-        c.beta = P.beta[slot];
-        c.L = P.L[slot];
-        c.o = mk3(r0.x, r0.y, r0.z);
-        c.prevPdf = r0.w;
-        c.d = mk3(r1.x, r1.y, r1.z);
-        const float4 pp = P.prevP[slot];
-        c.prevP = mk3(pp.x, pp.y, pp.z);
-        c.pixel = info.x;
-        c.region = info.z;
-        c.departed = info.w;
-        c.face = P.face[slot];
+        float4 r1;
+        loadPath(c, P, slot, passInc, r1);
         c.shPend = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         alive = shadeOne(c, P.hit[slot], P.count);
         P.L[slot] = c.L;
@@ -836,10 +846,51 @@ __global__ void clearCounts(uint32_t* c, int n) {
     if (threadIdx.x < unsigned(n)) c[threadIdx.x] = 0;
 }
 
-// Starts a chunk: queue 0 holds `count` paths, queue 1 none, no segments, inconsistencies or leaks yet.
-__global__ void setCount(uint32_t* c, unsigned long long* segments, uint32_t count) {
-    if (threadIdx.x < 4) c[threadIdx.x] = threadIdx.x == 0 ? count : 0u;
-    if (threadIdx.x == 0) *segments = 0;
+__device__ __forceinline__ void addSegments(unsigned long long* total, uint32_t segments) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) segments += __shfl_xor(segments, off);
+    if (__lane_id() == 0 && segments) atomicAdd(total, (unsigned long long)segments);
+}
+
+// The rest of every live path of queue q in one launch, a path a lane: the persistent form's loop from the
+// wavefront's records instead of the camera, with the same device functions, so each path's floats are those of
+// the rounds. Lanes k < per of a wave take a path each. Bound by the longest path's chain of segments (a round's
+// three launches cost about 27 µs whatever they do, and a path has up to 4·max_depth rounds); two waves a SIMD,
+// as the persistent form. Reset, pass and image of 3,072 paths of the glass caustic: 0.44 -> 0.21 ms (64x48).
+template <bool kContacts>
+__global__ __launch_bounds__(kBlock, 2) void drainKernel(DScene sc, Settings set, Paths P, int q, uint64_t passInc, int simple,
+                                                         uint32_t per) {
+    __shared__ uint32_t stack[48 * kBlock];
+    const uint32_t lane = __lane_id();
+    const uint32_t k = (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * per + lane;
+    uint32_t segments = 0;
+    if (lane < per && k < P.count[q]) {
+        const uint32_t slot = P.queue[q][k];
+        float4 r1;
+        ShadeCtx c{sc, set};
+        loadPath(c, P, slot, passInc, r1);
+        for (bool alive = true; alive;) {
+            Hit h;
+            const bool found = intersectContact<false, kContacts>(sc, c.o, c.d, __builtin_inff(), c.departed, c.face,
+                                                                  kNoBoundary, c.region, stack + threadIdx.x, kBlock, h);
+            ++segments;
+            const uint4 hraw = found ? make_uint4(__float_as_uint(h.t), h.boundary, h.face, h.slot)
+                                     : make_uint4(__float_as_uint(__builtin_inff()), kNoBoundary, 0u, kEmptyChild);
+            c.shPend = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            alive = shadeOne(c, hraw, P.count);
+            if (c.shPend.x != 0.0f || c.shPend.y != 0.0f || c.shPend.z != 0.0f || c.shPend.w != 0.0f) {
+                float Tr[NW];
+                const float4 lam = make_float4(c.wl.lambda[0], c.wl.lambda[1], c.wl.lambda[2], c.wl.lambda[3]);
+                if (shadowTransmittance<kContacts>(sc, c.shO, c.shD, c.shDist, c.shStart, c.shLightRegion, c.shExclude,
+                                                   c.shDeparted, c.shFace, lam, simple, stack + threadIdx.x, Tr))
+                    c.L = addShadow(c.L, c.shPend, Tr);
+            }
+            c.depth += 1;
+        }
+        P.L[slot] = c.L;
+        P.info[slot] = make_uint4(c.pixel, c.depth | (c.flags << 16), c.region, c.departed);
+    }
+    addSegments(P.segments, segments);
 }
 
 // ---------------------------------------------------------------- persistent form
@@ -978,12 +1029,6 @@ __device__ __forceinline__ uint32_t persistDrain(const DScene& sc, const Setting
     }
     flushFilm(a.film, accPix, acc);
     return segments;
-}
-
-__device__ __forceinline__ void addSegments(unsigned long long* total, uint32_t segments) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) segments += __shfl_xor(segments, off);
-    if (__lane_id() == 0 && segments) atomicAdd(total, (unsigned long long)segments);
 }
 
 // kWaves: the waves per SIMD the register allocation must allow (2: no spills; 3: more waves to
@@ -1939,8 +1984,8 @@ void allocPaths(owe_hip_renderer* r, uint32_t n) {
     P.shFace = devAlloc<uint32_t>(r, n);
     P.queue[0] = devAlloc<uint32_t>(r, n);
     P.queue[1] = devAlloc<uint32_t>(r, n);
-    P.count = devAlloc<uint32_t>(r, 4);
-    P.segments = devAlloc<unsigned long long>(r, 1);
+    P.count = devAlloc<uint32_t>(r, 6);  // the segments behind the counts: one copy reads both
+    P.segments = reinterpret_cast<unsigned long long*>(P.count + 4);
     r->capacity = n;
 }
 
@@ -1988,6 +2033,29 @@ void launchBounce(owe_hip_renderer* r, int q, uint32_t upper, uint64_t passInc) 
     hipLaunchKernelGGL(clearCounts, dim3{1}, dim3{64}, 0, r->stream, r->P.count + q, 1);
 }
 
+// The live count from which the rounds' remainder runs as one launch: eight paths to each lane the registers let
+// in (512 a compute unit). A round costs three launches and its compaction pays only while dead lanes would
+// idle a full chip. All rounds / drained from here (ms a pass): 12,288 paths of the glass caustic 0.43 / 0.16,
+// 98,304 of the pool 3.6 / 1.5 and of the telescope's room 5.0 / 1.3, 1,179,648 with the drain from 131,072, from
+// 524,288 or at once: pool 9.1, 7.7, 6.1, prism 0.85, 0.83, 0.64, room 6.9, 6.7, 7.0; 4,194,304 likewise: pool 18.1,
+// 17.9, 18.4, prism 2.5, 2.3, 3.0, room 19.2, 19.2, 26.6.
+uint64_t drainFrom(const owe_hip_renderer* r) { return uint64_t(r->computeUnits) * 512u * 8u; }
+
+void launchDrain(owe_hip_renderer* r, int q, uint32_t live, uint64_t passInc) {
+    // Few paths are spread over more waves, down to 8 a wave, while waves are free (8 a compute unit): a wave
+    // runs as long as its lanes' different ways together. 3,072 paths with 64 / 16 / 8 a wave: room 1.33 / 1.00 /
+    // 0.86 ms, pool 0.94 / 0.88 / 0.84, glass caustic 0.16 / 0.15 / 0.17.
+    uint32_t per = 8;
+    while (per < 64 && uint64_t(per) * uint32_t(r->computeUnits) * 8u < live) per *= 2;
+    const uint32_t waves = (live + per - 1) / per;
+    const dim3 grid{(waves + kBlock / 64 - 1) / (kBlock / 64)};
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3{kBlock}, 0, r->stream, r->dev, r->set, r->P, q, passInc, int(r->simpleShadows), per);
+    };
+    if (r->dev.contacts) go(drainKernel<true>);
+    else go(drainKernel<false>);
+}
+
 // Runs count paths: slots [0, count) with global path ids base + slot, or the (pixel, sample) lists.
 void runPaths(owe_hip_renderer* r, uint64_t base, uint32_t count, uint32_t spp, uint32_t pass, bool lists,
               double* perPath) {
@@ -2000,7 +2068,6 @@ void runPaths(owe_hip_renderer* r, uint64_t base, uint32_t count, uint32_t spp, 
     OWE_HIP_CHECK(hipGetLastError());
     bool generated = true;
     r->stats.paths += count;
-    const uint64_t segmentsBefore = r->stats.segments;
     // Rounds are enqueued in groups without waiting: each kernel reads its live count on the device.
     // The host reads the counters back once per group to stop, and the bound it knew (`upper`, the
     // live count at the last read) sizes the grids.
@@ -2010,8 +2077,11 @@ void runPaths(owe_hip_renderer* r, uint64_t base, uint32_t count, uint32_t spp, 
     const int maxRounds = 4 * r->set.maxDepth + 4;
     // Every round raises each live path's depth by one and no path outlives depth 4·maxDepth (null
     // crossings); the round limit only bounds the loop should that ever fail.
-    hipLaunchKernelGGL(setCount, dim3{1}, dim3{64}, 0, r->stream, r->P.count, r->P.segments, count);
     for (int round = 0; upper > 0 && round <= maxRounds;) {
+        if (!r->timing && upper <= drainFrom(r)) {
+            launchDrain(r, q, upper, passInc);
+            break;
+        }
         const int group = round < 2 ? 1 : r->roundsPerSync;
         for (int g = 0; g < group && round <= maxRounds; ++g, ++round) {
             if (r->dev.contacts) {
@@ -2038,21 +2108,18 @@ void runPaths(owe_hip_renderer* r, uint64_t base, uint32_t count, uint32_t spp, 
         generated = false;
         upper = hostCounts[q];
     }
-    r->stats.inconsistencies += hostCounts[2];
-    r->stats.leaks += hostCounts[3];
-    {
-        unsigned long long segs = 0;
-        OWE_HIP_CHECK(hipMemcpyAsync(&segs, r->P.segments, sizeof segs, hipMemcpyDeviceToHost, r->stream));
-        OWE_HIP_CHECK(hipStreamSynchronize(r->stream));
-        r->stats.segments = segmentsBefore + segs;
-    }
     timed(r, kSplat, [&] {
         hipLaunchKernelGGL(splatKernel, gridFor(count), dim3{kBlock}, 0, r->stream, r->set, r->P, count, r->invNWY, r->film,
                            perPath);
     });
     OWE_HIP_CHECK(hipGetLastError());
+    uint32_t last[6];
+    OWE_HIP_CHECK(hipMemcpyAsync(last, r->P.count, sizeof last, hipMemcpyDeviceToHost, r->stream));
+    OWE_HIP_CHECK(hipStreamSynchronize(r->stream));
+    r->stats.inconsistencies += last[2];
+    r->stats.leaks += last[3];
+    r->stats.segments += uint64_t(last[4]) | (uint64_t(last[5]) << 32);
     if (r->timing) {
-        OWE_HIP_CHECK(hipStreamSynchronize(r->stream));
         if (generated) collectTimes(r, {kGenerate});
         collectTimes(r, {kSplat});
     }

@@ -121,3 +121,48 @@ def test_shrinking_chunks_trace_every_path_once(cuda, width, height, spp, chunk,
     assert sa["paths"] == 2 * width * height * spp
     assert np.array_equal(a, b)
     assert sa == sb
+
+
+def _rounds_and_drain(make, st, spp, passes=2):
+    """(image, statistics) with every bounce a round of its own, as kernel timing asks for, and without timing."""
+    out = []
+    for rounds in (True, False):
+        r = render.Renderer(make(), st)
+        r.set_timing(rounds)
+        for _ in range(passes):
+            r.run_pass(spp)
+        out.append((r.resolve(), r.stats()))
+        r.close()
+    return out
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_drained_paths_equal_rounds_bit_for_bit(cuda, case):
+    make, st, spp = CASES[case]
+    (a, sa), (b, sb) = _rounds_and_drain(make, st, spp)
+    assert np.array_equal(a, b)
+    assert sa == sb
+
+
+# One path; a wave's first and last lane at 8 paths a wave; the step from 8 to 16 and from 32 to 64 paths a wave on
+# 2,048 waves; rounds that shrink to the drain (1,185,921 = 1,089² paths).
+@pytest.mark.parametrize("width,height,spp", [(1, 1, 1), (3, 3, 1), (128, 128, 1), (127, 129, 1), (113, 29, 5), (128, 128, 4),
+                                              (331, 99, 2), (1089, 1089, 1)])
+def test_drain_at_the_edges_of_its_split(cuda, width, height, spp):
+    (a, sa), (b, sb) = _rounds_and_drain(lambda: S.dispersion_prism_scene(width, height), S.settings(seed=8, **PRISM), spp, 1)
+    assert sa["paths"] == width * height * spp
+    assert np.array_equal(a, b)
+    assert sa == sb
+
+
+def test_drained_path_lists_equal_rounds(cuda):
+    st = S.settings(seed=10, **PRISM)
+    rng = np.random.default_rng(5)
+    pixel, sample = rng.integers(0, 64 * 64, 777, dtype=np.uint32), rng.integers(0, 16, 777, dtype=np.uint32)
+    out = []
+    for rounds in (True, False):
+        r = render.Renderer(S.dispersion_prism_scene(64, 64), st)
+        r.set_timing(rounds)
+        out.append(r.camera_paths(16, pixel, sample))
+        r.close()
+    assert np.array_equal(*out)
