@@ -2675,8 +2675,10 @@ int owe_hip_renderer_create(int device, const owe_scene* scene, const owe_render
             r->chunk = 4;
             r->regen = 32;
         }
-        r->scene = devAlloc<DScene>(r, 1);
-        OWE_HIP_CHECK(hipMemcpy(r->scene, &r->dev, sizeof r->dev, hipMemcpyHostToDevice));
+        if (r->integrator != OWE_INTEGRATOR_PATH && r->integrator != OWE_INTEGRATOR_SPPM) {
+            r->scene = devAlloc<DScene>(r, 1);
+            OWE_HIP_CHECK(hipMemcpy(r->scene, &r->dev, sizeof r->dev, hipMemcpyHostToDevice));
+        }
         *out = r;
     });
     if (st != OWE_HIP_OK && r) {
