@@ -254,22 +254,37 @@ __device__ __forceinline__ void walkNode(Walk& w, const WideNode* __restrict__ n
     walkPop(w, st, stride);
 }
 
-// Tests the first triangle of leaf reference w.cur and moves to its next one, or to the stack's top.
+// Tests the first two triangles of leaf reference w.cur (its only one where it has one) and moves to its next
+// ones, or to the stack's top. Both are loaded together: one wait for two tests, where one triangle a step
+// took 1.99 ms for 8,388,608 closest queries, 0.207 for 1,000,003 any-hit ones and 0.056 for 4,096 (with two 1.89, 0.199
+// and 0.053).
 template <bool kAny>
 __device__ __forceinline__ void walkTriangle(Walk& w, const TriRecord* __restrict__ tris, const WalkStack& st,
                                              uint32_t stride) {
-    const uint32_t slot = w.cur & kFirstMask;
+    constexpr int kMost = 2;
+    float4 v[kMost][3];
+    const uint32_t slot = w.cur & kFirstMask, more = (w.cur >> kCountShift) & 0xFu;  // triangles behind the first
     const float4* tr = reinterpret_cast<const float4*>(tris + slot);
-    const float4 a = tr[0], b = tr[1], c = tr[2];
-    float t;
-    if (hitTriangle(w.sh, w.o, w.d, mk3(a.x, a.y, a.z), mk3(b.x, b.y, b.z), mk3(c.x, c.y, c.z), w.tmin, w.hit.t, t)) {
-        w.hit = RayHit{t, slot};
-        if (kAny) {
-            w.cur = kEmptyChild;
-            return;
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        const uint32_t at = uint32_t(k) <= more ? uint32_t(k) : 0u;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[k][i] = tr[3 * at + i];
+    }
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        float t;
+        const f3 p0 = mk3(v[k][0].x, v[k][0].y, v[k][0].z), p1 = mk3(v[k][1].x, v[k][1].y, v[k][1].z),
+                 p2 = mk3(v[k][2].x, v[k][2].y, v[k][2].z);
+        if (uint32_t(k) <= more && hitTriangle(w.sh, w.o, w.d, p0, p1, p2, w.tmin, w.hit.t, t)) {
+            w.hit = RayHit{t, slot + uint32_t(k)};
+            if (kAny) {
+                w.cur = kEmptyChild;
+                return;
+            }
         }
     }
-    if (w.cur & (0xFu << kCountShift)) w.cur += 1u - (1u << kCountShift);  // one triangle fewer, from the next slot
+    if (more >= uint32_t(kMost)) w.cur += uint32_t(kMost) * (1u - (1u << kCountShift));  // fewer triangles, from a later slot
     else walkPop(w, st, stride);
 }
 
