@@ -332,10 +332,13 @@ __global__ __launch_bounds__(kCBlock) void causticForward(CArgs a) {
             for (int c = 0; c < 3; ++c) {
                 const int pi = ci + c - 1, pj = cj + b - 1;
                 if (pi < 0 || pj < 0 || pi >= int(a.pixels) || pj >= int(a.pixels)) continue;
-                // Scaling by 2³² is exact in float, so rounding there is rounding the exact product.
-                const unsigned long long units = (unsigned long long)rintf(w * wu[c] * wv[b] * float(kSplatUnits));
+                // Scaling by 2³² is exact in float, so rounding there is rounding the exact product. At the critical
+                // angle the transmittance can round below 0: a negative product adds nothing.
+                const float scaled = rintf(w * wu[c] * wv[b] * float(kSplatUnits));
+                if (!(scaled > 0.0f)) continue;
+                const unsigned long long units = (unsigned long long)scaled;
                 const uint32_t key = uint32_t(pj) * a.pixels + uint32_t(pi);
-                if (units > 0 && !table.add(key, units)) atomicAdd(a.acc + key, units);
+                if (!table.add(key, units)) atomicAdd(a.acc + key, units);
             }
     }
     __syncthreads();

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 
 from owe_hip import caustic as C
+from owe_hip.lens import ciddor_air
 from pyoracle import CausticOracle
 
 pytestmark = pytest.mark.gpu
@@ -214,4 +215,51 @@ def test_adjoint_of_wide_ranges_and_remainders(cuda, particles):
     assert torch.isfinite(got[:, 40:]).all() and (got[:, 40:].double() - inner).norm() <= 2e-5 * inner.norm()
     if particles >= 5000:
         assert not torch.isfinite(got[:, :40]).all()
+    c.close()
+
+
+@pytest.mark.parametrize("n", [1.2, 1.3, 1.4, 1.7])
+def test_exits_at_the_critical_angle_add_no_light(cuda, oracle, n):
+    """A tilted plane whose slope is the critical one, sin θ = 1/η: the float cos²θt = 1 − η² sin²θ takes its values
+    near 0, 0 among them, where the Fresnel amplitudes round past 1 and the transmittance below 0 (by up to
+    2.4e-7). cos θt stays below 0.02 there (sin θ varies by 1e-5 with the heights' rounding), so a particle
+    passes at most 4 cos θt < 0.13 of its weight, 0.26 of irradiance where the full weights give 1 to 2; a negative
+    weight taken for a large one is a whole unit of irradiance. (The cells at the slab's edge have other slopes.)"""
+    import torch
+
+    s = C.caustic_settings(particles=1 << 20, pixels=1024, thickness=0.06, wall_distance=0.1, wall_half=0.3)
+    s.medium.index_kind, s.medium.coeff_a[0] = 0, n
+    c = C.Caustic(s)
+    eta = n / ciddor_air(555.0)  # air's index varies by 7e-6 over the visible range
+    x = np.linspace(-s.slab_half, s.slab_half, s.nodes) / math.sqrt(eta * eta - 1)
+    H = np.broadcast_to(x, (s.nodes, s.nodes)).astype(np.float32)
+    E = forward(c, s, torch.tensor(H.copy(), device="cuda")).cpu().numpy().astype(np.float64)
+    Eo = CausticOracle(oracle, s).forward(H.astype(np.float64))
+    diff = np.abs(E - Eo).max()
+    print(f"index {n}: {E.sum():.3f} / {Eo.sum():.3f}, max {E.max():.3f} / {Eo.max():.3f}, max |ΔE| {diff:.3e}", flush=True)
+    assert diff < 0.26 + 1e-3 * Eo.max()
+    c.close()
+
+
+@pytest.mark.parametrize("kelvin", [110.0, 200.0, 300.0, 440.0])
+def test_adjoint_of_cool_suns(cuda, oracle, kelvin):
+    """Planck's exponent exceeds float's range over part of the visible range below 450 K and over all of it below
+    195 K; the weights are ratios and stay in range. The reddest particles carry the sums there."""
+    import torch
+
+    s = C.caustic_settings(nodes=64, pixels=128, particles=1 << 16, kelvin=kelvin)
+    c = C.Caustic(s)
+    H = torch.tensor(C.initial_heights(64, feature=16), device="cuda")
+    co = CausticOracle(oracle, s)
+    E, Eo = forward(c, s, H).cpu().numpy().astype(np.float64), co.forward(H.cpu().numpy().astype(np.float64))
+    # The exponent c2/(λT), up to 400, rounds by 2⁻²³ of itself twice: 1e-4 of a weight.
+    assert np.linalg.norm(E - Eo) <= 3e-4 * np.linalg.norm(Eo)
+    T = torch.tensor(C.target(s), device="cuda")
+    g = adjoint(c, s, H, T).cpu().numpy().ravel().astype(np.float64)
+    assert np.isfinite(g).all()
+    nodes = np.argsort(-np.abs(g))[:: 64][:16]
+    fd = co.fd(H.cpu().numpy().astype(np.float64), T.cpu().numpy().astype(np.float64), nodes, 1e-9)
+    rel = np.linalg.norm(g[nodes] - fd) / np.linalg.norm(fd)
+    print(f"{kelvin} K: adjoint against fp64 differences {rel:.2e}", flush=True)
+    assert rel < 1e-3
     c.close()
