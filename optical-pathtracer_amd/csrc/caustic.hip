@@ -50,7 +50,9 @@ struct CArgs {
     float perCell, perPix;   // 1 / cell, 1 / pix
     uint64_t particles, seed, pass;
     DMedium slab, air;
-    float kelvin, invY;      // sun temperature; 1 / ∫ B ȳ over 360–830 nm
+    // The sun's B(λ) / ∫ B ȳ = sunScale e / (λ⁵ (1 − e sunRef)) with e = exp(sunAt − sunC2 / λ), λ in µm: the exponent is
+    // taken from that of 555 nm (sunAt; sunRef = exp(−sunAt)), since a cool sun's own leaves float's range.
+    float sunScale, sunC2, sunAt, sunRef;
     float tileArea;          // a tile's area / pixel area: with a tile's particle count, irradiance per unit weight
     uint32_t tiles;          // tiles per side (a power of two)
     uint32_t tileShift;      // log2 of all tiles
@@ -194,15 +196,16 @@ __device__ __forceinline__ Particle drawParticle(const CArgs& a, uint64_t i) {
     q.y = -a.slabHalf + (float(mortonHalf(uint32_t(t >> 1))) + u2) * side;
     q.eta = quick(mediumIndex(a.slab, lambda), mediumIndex(a.air, lambda));
     const float r = quick(q.eta - 1.0f, q.eta + 1.0f);  // the entry's Fresnel amplitude at normal incidence
-    // B(λ) ȳ(λ) / pdf over the sun's ∫ B ȳ, one quotient: planckF and cieXYZ's ȳ.
+    // B(λ) ȳ(λ) / pdf over the sun's ∫ B ȳ, one quotient of normal numbers for any sun above 100 K (|e's exponent| < 86
+    // toward the red; toward the blue e may vanish): Planck's law and cieXYZ's ȳ.
     const float l = lambda * 1e-3f, l2 = l * l;
     auto lobe = [&](float mu, float below, float above) {
         const float u = (lambda - mu) * (lambda < mu ? below : above);
         return expf(-0.5f * u * u);
     };
     const float y = 0.821f * lobe(568.8f, 1.0f / 46.9f, 1.0f / 40.5f) + 0.286f * lobe(530.9f, 1.0f / 16.3f, 1.0f / 31.1f);
-    const float planckDen = l2 * l2 * l * (expf(quick(1.438776877e4f, l * a.kelvin)) - 1.0f);
-    q.weight = quick(1e6f * 1.191042972e8f * a.invY * a.tileArea * y * (1.0f - r * r), planckDen * pdf * float(count));
+    const float e = expf(a.sunAt - quick(a.sunC2, l));
+    q.weight = quick(a.sunScale * a.tileArea * y * (1.0f - r * r) * e, l2 * l2 * l * (1.0f - e * a.sunRef) * pdf * float(count));
     return q;
 }
 
@@ -540,7 +543,6 @@ CArgs makeArgs(const owe_caustic_settings& s) {
     owe_medium air{};
     air.index_kind = OWE_INDEX_CIDDOR;
     a.air = toDevMedium(air);
-    a.kelvin = float(s.sun_kelvin);
     // ∫ B ȳ dλ over 360–830 nm (composite Simpson, 0.5 nm).
     const int n = 940;
     const double hh = 470.0 / n;
@@ -549,7 +551,10 @@ CArgs makeArgs(const owe_caustic_settings& s) {
         const double l = 360.0 + k * hh;
         sum += planck(l, s.sun_kelvin) * cieYHost(l) * ((k & 1) ? 4 : 2);
     }
-    a.invY = float(1.0 / (sum * hh / 3));
+    a.sunC2 = float(1.438776877e4 / s.sun_kelvin);
+    a.sunAt = float(1.438776877e4 / (0.555 * s.sun_kelvin));
+    a.sunRef = float(std::exp(-double(a.sunAt)));
+    a.sunScale = float(1e6 * 1.191042972e8 * std::exp(-double(a.sunAt)) / (sum * hh / 3));
     const double pix = 2 * s.wall_half / s.pixels;
     a.tiles = causticTiles(s.particles);
     while ((uint64_t(1) << a.tileShift) < uint64_t(a.tiles) * a.tiles) ++a.tileShift;

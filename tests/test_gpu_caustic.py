@@ -239,3 +239,27 @@ def test_exits_at_the_critical_angle_add_no_light(cuda, oracle, n):
     print(f"index {n}: {E.sum():.3f} / {Eo.sum():.3f}, max {E.max():.3f} / {Eo.max():.3f}, max |ΔE| {diff:.3e}", flush=True)
     assert diff < 0.26 + 1e-3 * Eo.max()
     c.close()
+
+
+@pytest.mark.parametrize("kelvin", [110.0, 200.0, 300.0, 440.0])
+def test_adjoint_of_cool_suns(cuda, oracle, kelvin):
+    """Planck's exponent exceeds float's range over part of the visible range below 450 K and over all of it below
+    195 K; the weights are ratios and stay in range. The reddest particles carry the sums there."""
+    import torch
+
+    s = C.caustic_settings(nodes=64, pixels=128, particles=1 << 16, kelvin=kelvin)
+    c = C.Caustic(s)
+    H = torch.tensor(C.initial_heights(64, feature=16), device="cuda")
+    co = CausticOracle(oracle, s)
+    E, Eo = forward(c, s, H).cpu().numpy().astype(np.float64), co.forward(H.cpu().numpy().astype(np.float64))
+    # The exponent c2/(λT), up to 400, rounds by 2⁻²³ of itself twice: 1e-4 of a weight.
+    assert np.linalg.norm(E - Eo) <= 3e-4 * np.linalg.norm(Eo)
+    T = torch.tensor(C.target(s), device="cuda")
+    g = adjoint(c, s, H, T).cpu().numpy().ravel().astype(np.float64)
+    assert np.isfinite(g).all()
+    nodes = np.argsort(-np.abs(g))[:: 64][:16]
+    fd = co.fd(H.cpu().numpy().astype(np.float64), T.cpu().numpy().astype(np.float64), nodes, 1e-9)
+    rel = np.linalg.norm(g[nodes] - fd) / np.linalg.norm(fd)
+    print(f"{kelvin} K: adjoint against fp64 differences {rel:.2e}", flush=True)
+    assert rel < 1e-3
+    c.close()
