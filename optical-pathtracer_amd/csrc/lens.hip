@@ -475,11 +475,11 @@ __global__ __launch_bounds__(kLensBlock) void lensKernel(LensArgs a) {
             // The ray's spot terms in float (B = d_xy / d_z, A at z = 0 or the angles), summed in
             // double. An afocal spot's variance is 10⁻⁴ and less of its mean square, so its y angles
             // are taken relative to the angle refA of a slope refB near them, where float keeps their digits:
-            // atan b = refA + atan((b − refB) / (1 + b refB)).
+            // the argument of (1 + i b)(1 − i refB), in (−π, π), for a ray on either side of the axis.
             const float iz = quick(1.0f, d.z);
             const float bx = d.x * iz, by = d.y * iz;
             const float ax = L.afocal ? atanf(bx) : p.x - bx * p.z;
-            const float ay = L.afocal ? atanf((by - L.refB) / (1.0f + by * L.refB)) : p.y - by * p.z;
+            const float ay = L.afocal ? atan2f(d.y - L.refB * d.z, d.z + L.refB * d.y) : p.y - by * p.z;
             if (kGrad) {
 #pragma unroll
                 for (int kp = 0; kp < kGroup; ++kp) {

@@ -230,3 +230,59 @@ def test_conic_roots_of_every_form_match_oracle(cuda, oracle, field):
     b.close()
     print(f"field {field}: {total} rays arrive on both, {flips} flips, {far} beyond the bound", flush=True)
     assert total > 20 * 2048 and flips <= total // 1000 and far <= total // 100
+
+
+@pytest.mark.parametrize("asphere", [(3e5, -4e5, 1e5, -4e5), (0.0, -4e5, 3e5, -1e5)])
+@pytest.mark.parametrize("params", [0, 2])
+def test_afocal_angles_on_both_sides_of_the_axis(cuda, oracle, asphere, params):
+    """Two aspheric plates (afocal, magnification 1) at 60 degrees: some rays leave more than a right angle from the
+    paraxial apparent direction. The sums of angles are the oracle's up to rays that only one of the two loses
+    (an angle below π/2 each) and 1e-6 a ray, the direction's error in this file's other tests times the plates' steepness."""
+    rows = [L.Surface(math.inf, t, g, sd, A=(a,), stop=k == 0)
+            for k, (t, g, sd, a) in enumerate(zip((4.0, 2.0, 4.0, 4.0), ("N-SF11", "air", "N-SF11", "air"),
+                                                  (8.0, 12.0, 14.0, 16.0), asphere))]
+    p = L.Prescription(rows, rays=4096)
+    b = L.LensBatch([p], L.c_settings(field_deg=60.0, pixels=0))
+    if params:
+        b.set_params([(0, L.PARAM_A4), (3, L.PARAM_A4)][:params])
+    b.run()
+    per, mom, _ = b.results()
+    lo = LensOracle(oracle, [p], field_deg=60.0)
+    assert per[0]["afocal"]
+    strays = 0
+    for w, lam in enumerate(L.FRAUNHOFER7):
+        ray = lo.trace(0, lam, np.arange(p.rays, dtype=np.uint64))
+        ray = ray[ray[:, 6] > 0]
+        strays += int((ray[:, 4] / ray[:, 5] * math.tan(math.radians(60.0)) < -1).sum())
+        want, got = lo.moments(0, lam)[0], mom[0, w]
+        flips = abs(want[0] - got[0]) + max(2, p.rays // 2000)
+        print(f"line {w}: {int(got[0])} rays, Σ|Δ| {np.abs(got[1:3] - want[1:3])}", flush=True)
+        assert (np.abs(got[1:3] - want[1:3]) <= flips * math.pi / 2 + 1e-6 * want[0]).all()
+        assert abs(got[5] - want[5]) <= flips * (math.pi / 2) ** 2 + 3e-6 * want[0]
+    assert strays > 500
+    if params:
+        # d(angular rms)/dθ from 64-bit differences of the rays that arrive on both sides.
+        idx = np.arange(p.rays, dtype=np.uint64)
+        which = [(0, L.PARAM_A4), (3, L.PARAM_A4)]
+
+        def rms(delta):
+            rays = [lo.trace_perturbed(0, lam, which, delta, idx) for lam in L.FRAUNHOFER7]
+            return np.concatenate([r[:, 3:7] for r in rays])
+
+        grads = b.gradients()[0]
+        for k, step in enumerate((0.1, 0.1)):
+            lo_, hi = (rms([s * step if j == k else 0.0 for j in range(2)]) for s in (-1, 1))
+            ok = (lo_[:, 3] > 0) & (hi[:, 3] > 0)
+
+            def value(r):
+                bxy = r[ok, :2] / r[ok, 2:3]
+                return math.sqrt(((np.arctan(bxy) - np.arctan(bxy.mean(0))) ** 2).sum(1).mean())
+
+            fd = (value(hi) - value(lo_)) / (2 * step)
+            # A ray that leaves a surface at grazing has a derivative of 1 / cos θt, 10⁴ times the others', and cos²θt
+            # rounds by 1.2e-7: at cos θt = 1e-3 its share of the mean is off by a tenth (the largest share
+            # alone exceeds the whole of the first design's first derivative).
+            share = np.abs(np.arctan(hi[ok, 1] / hi[ok, 2]) - np.arctan(lo_[ok, 1] / lo_[ok, 2])).max() / (2 * step) / ok.sum()
+            print(f"parameter {k}: {grads[k]:.6e}, 64-bit difference {fd:.6e}, largest share {share:.1e}", flush=True)
+            assert abs(grads[k] - fd) <= 2e-3 * abs(fd) + 0.1 * share
+    b.close()
