@@ -32,9 +32,11 @@ __host__ __device__ inline float len3(f3 a) { return sqrtf(dot3(a, a)); }
 __host__ __device__ inline f3 norm3(f3 a) { return a / len3(a); }
 __host__ __device__ inline float comp(f3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 
-// Quotients and roots of normal values to about an ulp: the hardware's estimate and one Newton step (two
-// for a double quotient's reciprocal), where the correctly rounded forms take 11 to 20 instructions and
-// their last half ulp is far below the rounding of the coordinates they lead to.
+// Quotients and roots of normal values to about an ulp: the hardware's estimate and one Newton step (a double
+// quotient: two for the reciprocal and one for the quotient), where the correctly rounded forms take 11 to 20
+// instructions and their last half ulp is far below the rounding of the coordinates they lead to. A quotient's
+// denominator is neither 0, subnormal nor infinite and its reciprocal not subnormal: those give NaN or infinity,
+// also where the true quotient is 0.
 __device__ __forceinline__ float quick(float num, float den) {
     const float r = __builtin_amdgcn_rcpf(den);
     return num * (r * (2.0f - den * r));
@@ -49,7 +51,7 @@ __device__ __forceinline__ float invSqrt(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
     return y * (1.5f - 0.5f * x * y * y);
 }
-__device__ __forceinline__ float quickSqrt(float x) {  // 0 for x ≤ 0
+__device__ __forceinline__ float quickSqrt(float x) {  // 1e-15 for x ≤ 1e-30, also below 0 (double: 1e-140, 1e-280)
     x = fmaxf(x, 1e-30f);
     const float y = __builtin_amdgcn_rsqf(x), v = x * y;
     return v + 0.5f * y * (x - v * v);

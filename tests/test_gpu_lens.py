@@ -286,3 +286,26 @@ def test_afocal_angles_on_both_sides_of_the_axis(cuda, oracle, asphere, params):
             print(f"parameter {k}: {grads[k]:.6e}, 64-bit difference {fd:.6e}, largest share {share:.1e}", flush=True)
             assert abs(grads[k] - fd) <= 2e-3 * abs(fd) + 0.1 * share
     b.close()
+
+
+def test_rays_share_no_error_and_weights_keep_their_digits(cuda, oracle):
+    """Every ray reaches the first vertex plane after the same distance of 5 to 7 cm (ulp 3.7e-9 m) at the same slope
+    0.0087: correctly rounded it moves a lens's rays by up to 1.6e-11 m in y, of either sign, so the mean over 48
+    lenses lies below 1e-11, and one ulp in all of them is 3.3e-11. A weight near 0.85 after three faces, T − T R at
+    each, rounds by at most half an ulp (3e-8) at each, 1.7e-8 rms, and its R ≈ 0.05 by a few
+    ulps of 3.7e-9, so its rms error lies below 3.5e-8 (the indices' own rounding included)."""
+    lenses = L.seeded_achromats(48, seed=77, rays_min=20000, rays_max=40000)
+    b = L.LensBatch(lenses, L.c_settings(pixels=0))
+    lo = LensOracle(oracle, lenses)
+    dy, dT = [], []
+    for li, p in enumerate(lenses):
+        idx = np.arange(p.rays, dtype=np.uint64)
+        g, c = b.trace(li, 3, idx), lo.trace(li, L.FRAUNHOFER7[3], idx)
+        both = (g[:, 6] > 0) & (c[:, 6] > 0)
+        dy.append((g - c)[both, 1])
+        dT.append((g - c)[both, 6])
+    b.close()
+    dy, dT = np.concatenate(dy), np.concatenate(dT)
+    print(f"{len(dy)} rays: mean error of y {dy.mean():.2e} m, rms of the weight {np.sqrt((dT**2).mean()):.2e}", flush=True)
+    assert abs(dy.mean()) < 1e-11
+    assert np.sqrt((dT**2).mean()) < 3.5e-8
