@@ -751,8 +751,11 @@ T* lensAlloc(owe_hip_lens_batch* b, size_t n) {
     return static_cast<T*>(p);
 }
 
-// The work items of each lens for the current raysPerItem.
+// The work items of each lens of raysPerItem rays or, since a block traces an item, of the next whole number of
+// rays to each of its threads: items of 64 rays would leave three waves of four idle (16 Gregorians with four
+// derivatives 0.363 ms, with 256 rays 0.122; the form with an item to a wave 0.303 and 0.212).
 void layoutItems(owe_hip_lens_batch* b, uint32_t raysPerItem) {
+    raysPerItem = (raysPerItem + kLensBlock - 1) / kLensBlock * kLensBlock;
     uint64_t base = 0;
     for (DLensInfo& L : b->info) {
         L.itemBase = base;

@@ -309,3 +309,25 @@ def test_rays_share_no_error_and_weights_keep_their_digits(cuda, oracle):
     print(f"{len(dy)} rays: mean error of y {dy.mean():.2e} m, rms of the weight {np.sqrt((dT**2).mean()):.2e}", flush=True)
     assert abs(dy.mean()) < 1e-11
     assert np.sqrt((dT**2).mean()) < 3.5e-8
+
+
+def test_items_of_fewer_rays_than_threads_cost_no_more(cuda):
+    """A block traces an item: 64, 128, 192 and 320 rays take the time of the next multiple of 256 (within a third, the
+    spread of single launches of 0.1 ms being a tenth) and give its results."""
+    b = L.LensBatch(L.gregorian_variants(16, 60, 5), L.c_settings(field_deg=0.05, pixels=0))
+    b.set_params([(0, L.PARAM_CURVATURE), (1, L.PARAM_CONIC)])
+
+    def run(rays):
+        b.set_shape(3, rays)
+        ms = []
+        for _ in range(9):
+            b.run()
+            ms.append(b.last_ms())
+        return float(np.median(ms)), b.results()[1], b.gradients()
+
+    for rays, whole in ((64, 256), (128, 256), (192, 256), (320, 512)):
+        (t, m, g), (tw, mw, gw) = run(rays), run(whole)
+        print(f"items of {rays}: {t:.3f} ms, of {whole}: {tw:.3f} ms", flush=True)
+        assert np.allclose(m, mw, rtol=1e-12, atol=1e-9) and np.allclose(g, gw, rtol=1e-9, atol=1e-9 * np.abs(gw).max())
+        assert t <= tw * 4 / 3
+    b.close()
