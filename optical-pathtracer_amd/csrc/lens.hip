@@ -38,6 +38,7 @@ namespace owehip {
 namespace {
 
 constexpr int kLensBlock = 256;
+constexpr int kResidentBlocks = 3;  // blocks to a compute unit that registers and LDS hold
 constexpr double kHistScale = 4294967296.0;  // 2^32 units of weight per unit
 // A block's bin table: open addressing over kHashSlots (bin, sum) pairs, at most kHashProbes probes
 // before an add goes straight to HBM. An aberrated lens's five planes touch 1,000 bins and more: a table
@@ -734,7 +735,7 @@ struct owe_hip_lens_batch {
     double* gridScale = nullptr;  // irradiance per unit of a lens's bins, and the grids (made by the first results)
     float* irradiance = nullptr;
     int computeUnits = 256;
-    int blocksPerCU = 3;  // what registers and LDS hold
+    int blocksPerCU = kResidentBlocks;
     hipEvent_t ev[2] = {nullptr, nullptr};
     double lastMs = 0;
     bool ran = false;
@@ -773,7 +774,7 @@ void layoutItems(owe_hip_lens_batch* b, uint32_t raysPerItem) {
 uint32_t defaultItem(const owe_hip_lens_batch* b) {
     uint64_t rays = 0;
     for (const DLensInfo& L : b->info) rays += L.rays * b->args.nLambda;
-    const uint64_t per = rays / (uint64_t(b->computeUnits) * uint64_t(b->blocksPerCU) * 8);
+    const uint64_t per = rays / (uint64_t(b->computeUnits) * uint64_t(kResidentBlocks) * 8);
     return uint32_t(std::clamp<uint64_t>((per + kLensBlock - 1) / kLensBlock * kLensBlock, kLensBlock, 4096));
 }
 
@@ -1117,8 +1118,13 @@ int owe_hip_lens_batch_autotune(owe_hip_lens_batch* b, double* best_ms) {
             layoutItems(b, c.rays);
             return runOnce(b);
         };
-        for (int blocks : {1, 2, 4, 8})
-            for (uint32_t rays : {256u, 1024u, 4096u, 16384u}) {
+        // Up to the resident blocks (48 achromats with three, four and eight 1.023, 1.016 and 1.018 ms; six small lenses with
+        // two, four and eight 0.021, 0.027 and 0.037), and the batch's own item.
+        std::vector<uint32_t> items{256u, 1024u, 4096u, 16384u};
+        const uint32_t own = defaultItem(b);
+        if (std::find(items.begin(), items.end(), own) == items.end()) items.push_back(own);
+        for (int blocks = 1; blocks <= kResidentBlocks; ++blocks)
+            for (uint32_t rays : items) {
                 cands.push_back({blocks, rays, 0.0});
                 cands.back().ms = run(cands.back());
             }

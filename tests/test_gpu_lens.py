@@ -331,3 +331,22 @@ def test_items_of_fewer_rays_than_threads_cost_no_more(cuda):
         assert np.allclose(m, mw, rtol=1e-12, atol=1e-9) and np.allclose(g, gw, rtol=1e-9, atol=1e-9 * np.abs(gw).max())
         assert t <= tw * 4 / 3
     b.close()
+
+
+@pytest.mark.parametrize("lenses,rays_max", [(1, 4096), (6, 40_000), (24, 60_000)])
+def test_autotune_takes_no_slower_shape_than_the_batchs_own(cuda, lenses, rays_max):
+    """The batch's own shape is among those tried, so the tuned one is no slower but for the spread of a launch (a tenth)."""
+    b = L.LensBatch(L.seeded_achromats(lenses, seed=3, rays_min=2048, rays_max=rays_max))
+
+    def median():
+        ms = []
+        for _ in range(15):
+            b.run()
+            ms.append(b.last_ms())
+        return float(np.median(ms))
+
+    own, best = median(), b.autotune()
+    tuned = median()
+    print(f"{lenses} lenses: own {own:.4f} ms, tuned {tuned:.4f} (as timed by the tuner {best:.4f})", flush=True)
+    assert tuned <= 1.1 * own
+    b.close()
