@@ -3085,7 +3085,9 @@ uint64_t fnvVec(uint64_t h, const std::vector<T>& v) {
 
 // The cache key: the device (architecture, compute units), the form, the pass size and the scene
 // as flattened for the device (every table the kernels read, the hierarchy's size), the settings
-// that change the work (integrator, spectral mode, depths) — not the seed.
+// that change the work (integrator, spectral mode, depths) — not the seed. The number in the name grows with
+// kernels whose best shapes differ (2: chunks shrink, the last paths of the wavefront are drained, the refilling
+// particle kernel is held to two waves per SIMD), so shapes tuned for the older ones are not taken.
 std::string tuningKey(const owe_hip_renderer* r, int spp) {
     hipDeviceProp_t p;
     OWE_HIP_CHECK(hipGetDeviceProperties(&p, r->device));
@@ -3108,7 +3110,7 @@ std::string tuningKey(const owe_hip_renderer* r, int spp) {
     h = fnvVec(h, r->host.bvh.tris);
     h = fnv1a(h, &r->host.obs, sizeof r->host.obs);
     char buf[40];
-    std::snprintf(buf, sizeof buf, "owe-hip-tune-1-%016llx", static_cast<unsigned long long>(h));
+    std::snprintf(buf, sizeof buf, "owe-hip-tune-2-%016llx", static_cast<unsigned long long>(h));
     return buf;
 }
 

@@ -58,3 +58,26 @@ def test_wavefront_tunes_paths_in_flight(cuda):
     ref = render.Renderer(sc, st)
     ref.run_pass(16)
     assert np.array_equal(w.resolve(), ref.resolve())
+
+
+def test_records_of_older_kernels_are_not_taken(cuda, tmp_path):
+    """A record under an older key's name (the shapes of kernels since replaced) is no hit."""
+    path = tmp_path / "tuning.txt"
+    render.set_tuning_cache(path)
+    try:
+        sc, st = S.dispersion_prism_scene(32, 32), S.settings(seed=3, **PRISM)
+
+        def tuned():
+            r = render.Renderer(sc, st)
+            r.set_mode(render.Renderer.PERSISTENT)
+            r.autotune(4)
+            return r
+
+        assert not tuned().tuning()["from_cache"]
+        assert tuned().tuning()["from_cache"]
+        key, rest = path.read_text().split(" ", 1)
+        path.write_text("owe-hip-tune-1-" + key.rsplit("-", 1)[1] + " " + rest)
+        assert not tuned().tuning()["from_cache"]
+        assert path.read_text().splitlines()[1].split(" ", 1)[0] == key
+    finally:
+        render.set_tuning_cache(None)
