@@ -586,9 +586,10 @@ __global__ void lensBegin(LensArgs a, size_t nMoments, size_t nHist, size_t nGra
 // The irradiance grids from the weights' integers, each lens's scaled by its own factor. On the host the
 // copy of 8-byte bins to pageable memory and their conversion took 12 ms of a 15 ms run with results
 // (64 lenses, five planes of 128²); a float is all that leaves the card now, and that run takes 5.8 ms.
-__global__ void lensResolve(const unsigned long long* hist, const double* scale, float* out, uint32_t lensBins, size_t n) {
+__global__ void lensResolve(const unsigned long long* hist, const double* scale, float* out, uint32_t lensBins, size_t first,
+                            size_t n) {
     for (size_t k = size_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n; k += size_t(gridDim.x) * blockDim.x)
-        out[k] = float(double(hist[k]) * scale[k / lensBins]);
+        out[k] = float(double(hist[first + k]) * scale[(first + k) / lensBins]);
 }
 
 // Resets the item counter between the gradient passes of one run.
@@ -732,8 +733,8 @@ struct owe_hip_lens_batch {
     owe_lens_batch_settings settings{};
     LensArgs args{};
     size_t nMoments = 0, nHist = 0, nGrads = 0;
-    double* gridScale = nullptr;  // irradiance per unit of a lens's bins, and the grids (made by the first results)
-    float* irradiance = nullptr;
+    double* gridScale = nullptr;    // irradiance per unit of a lens's bins (0: an afocal lens has no grid)
+    float* irradiance = nullptr;    // up to kResolveBins of the grids on their way to the host
     int computeUnits = 256;
     int blocksPerCU = kResidentBlocks;
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -751,6 +752,10 @@ T* lensAlloc(owe_hip_lens_batch* b, size_t n) {
     b->allocations.push_back(p);
     return static_cast<T*>(p);
 }
+
+// The grids become floats in pieces of up to 64 MiB, made with the batch: results cannot fail for memory after a
+// run, and the largest batches need no second copy of their grids.
+constexpr size_t kResolveBins = size_t(1) << 24;
 
 // The work items of each lens of raysPerItem rays or, since a block traces an item, of the next whole number of
 // rays to each of its threads: items of 64 rays would leave three waves of four idle (16 Gregorians with four
@@ -972,6 +977,20 @@ int owe_hip_lens_batch_create(int device, const owe_medium* media, uint32_t n_me
         a.moments = lensAlloc<double>(b, b->nMoments);
         b->nHist = size_t(n_lenses) * a.planes * a.pixels * a.pixels;
         a.hist = lensAlloc<unsigned long long>(b, b->nHist);
+        if (b->nHist > 0) {
+            // Unit irradiance across the beam: each ray carries π r² cos θ / (rays · nλ) of flux.
+            std::vector<double> scale(n_lenses, 0.0);
+            for (uint32_t li = 0; li < n_lenses; ++li) {
+                const DLensInfo& I = b->info[li];
+                if (!(I.detHalf > 0)) continue;
+                const double pix = 2.0 * I.detHalf / a.pixels;
+                scale[li] = 3.14159265358979323846 * I.rEP * I.rEP * 0.999 * 0.999 * a.dirZ /
+                            (double(I.rays) * nw * kHistScale * pix * pix);
+            }
+            b->gridScale = lensAlloc<double>(b, n_lenses);
+            OWE_HIP_CHECK(hipMemcpy(b->gridScale, scale.data(), n_lenses * sizeof(double), hipMemcpyHostToDevice));
+            b->irradiance = lensAlloc<float>(b, std::min(b->nHist, kResolveBins));
+        }
         b->nGrads = 0;
         a.grads = lensAlloc<double>(b, size_t(n_lenses) * nw * OWE_LENS_MAX_PARAMS * kGradSums);
         a.nParams = 0;
@@ -1191,26 +1210,14 @@ int owe_hip_lens_batch_results(owe_hip_lens_batch* b, owe_lens_result* lenses, d
             }
         }
         if (irradiance && px > 0) {
-            if (!b->irradiance) {
-                // Unit irradiance across the beam: each ray carries π r² cos θ / (rays · nλ) of flux.
-                std::vector<double> scale(nl, 0.0);  // 0: an afocal lens has no grid
-                for (uint32_t li = 0; li < nl; ++li) {
-                    const DLensInfo& I = b->info[li];
-                    if (!(I.detHalf > 0)) continue;
-                    const double pix = 2.0 * I.detHalf / px;
-                    scale[li] = 3.14159265358979323846 * I.rEP * I.rEP * 0.999 * 0.999 * b->args.dirZ /
-                                (double(I.rays) * nw * kHistScale * pix * pix);
-                }
-                double* s = lensAlloc<double>(b, nl);
-                OWE_HIP_CHECK(hipMemcpy(s, scale.data(), nl * sizeof(double), hipMemcpyHostToDevice));
-                b->gridScale = s;
-                b->irradiance = lensAlloc<float>(b, b->nHist);
+            for (size_t at = 0; at < b->nHist; at += kResolveBins) {
+                const size_t n = std::min(kResolveBins, b->nHist - at);
+                hipLaunchKernelGGL(lensResolve, dim3{2048}, dim3{256}, 0, b->stream, b->args.hist, b->gridScale,
+                                   b->irradiance, uint32_t(b->args.planes * px * px), at, n);
+                OWE_HIP_CHECK(hipGetLastError());
+                OWE_HIP_CHECK(hipMemcpyAsync(irradiance + at, b->irradiance, n * sizeof(float), hipMemcpyDeviceToHost, b->stream));
+                OWE_HIP_CHECK(hipStreamSynchronize(b->stream));
             }
-            hipLaunchKernelGGL(lensResolve, dim3{2048}, dim3{256}, 0, b->stream, b->args.hist, b->gridScale, b->irradiance,
-                               uint32_t(b->args.planes * px * px), b->nHist);
-            OWE_HIP_CHECK(hipGetLastError());
-            OWE_HIP_CHECK(hipMemcpyAsync(irradiance, b->irradiance, b->nHist * sizeof(float), hipMemcpyDeviceToHost, b->stream));
-            OWE_HIP_CHECK(hipStreamSynchronize(b->stream));
         }
     });
 }

@@ -1866,7 +1866,7 @@ struct owe_hip_renderer {
     uint32_t queueCapacity = 0;  // wavefront paths in flight per chunk (≤ capacity; tuned)
     bool tunedFromCache = false;
     unsigned long long* film = nullptr;
-    double* resolved = nullptr;  // resolve's image (made by the first)
+    double* resolved = nullptr;  // resolve's image: made with the renderer, so no image can fail for memory after its render
     double* perPath = nullptr;
     uint32_t* pathPixels = nullptr;
     uint32_t* pathSamples = nullptr;
@@ -2524,8 +2524,9 @@ int owe_hip_renderer_create(int device, const owe_scene* scene, const owe_render
             r->invNWY = float(1.0 / (NW * (sum * hh / 3)));
         }
         const uint64_t pixels = uint64_t(h.obs.width) * uint64_t(h.obs.height);
-        r->film = devAlloc<unsigned long long>(r, 3 * pixels);
+        r->film = devAlloc<unsigned long long>(r, 6 * pixels);  // and resolve's image behind it
         OWE_HIP_CHECK(hipMemset(r->film, 0, 3 * pixels * sizeof(unsigned long long)));
+        r->resolved = reinterpret_cast<double*>(r->film + 3 * pixels);
         if (r->integrator == OWE_INTEGRATOR_PATH || r->integrator == OWE_INTEGRATOR_HYBRID) {
             // The wavefront form's path slots are allocated at its first pass (runPaths): a renderer
             // that only runs the persistent form, or only as a batch member, never holds them. The
@@ -2829,7 +2830,6 @@ int owe_hip_renderer_resolve(owe_hip_renderer* r, double* xyz) {
         require(r != nullptr && xyz != nullptr, "null argument");
         OWE_HIP_CHECK(hipSetDevice(r->device));
         const size_t n = 3 * size_t(r->host.obs.width) * size_t(r->host.obs.height);
-        if (!r->resolved) r->resolved = devAlloc<double>(r, n);
         // Camera samples ÷ samples a pixel; particle splats ÷ particles emitted (gpu_renderer_film.cpp:17-20).
         const double norm = r->totalSpp > 0 ? 1.0 / (kFilmScale * double(r->totalSpp)) : 0.0;
         const double lightNorm = r->particleCount > 0 ? 1.0 / r->particleCount : 0.0;

@@ -350,3 +350,25 @@ def test_autotune_takes_no_slower_shape_than_the_batchs_own(cuda, lenses, rays_m
     print(f"{lenses} lenses: own {own:.4f} ms, tuned {tuned:.4f} (as timed by the tuner {best:.4f})", flush=True)
     assert tuned <= 1.1 * own
     b.close()
+
+
+def test_results_take_no_memory_and_pieces_of_the_grids_join(cuda):
+    """30 million bins leave the device in two pieces: the same lens gives the same grids in each place of the batch, one
+    of which lies across the join, and the first results allocate nothing."""
+    import torch
+
+    lenses = [L.DOUBLET] * 5
+    b = L.LensBatch(lenses, L.c_settings(planes=6, pixels=1000, half_size=3e-3))
+    b.run()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    _, mom, irr = b.results(irradiance=True)
+    assert torch.cuda.mem_get_info()[0] == free
+    one = L.LensBatch(lenses[:1], L.c_settings(planes=6, pixels=1000, half_size=3e-3))
+    one.run()
+    alone = one.results(irradiance=True)[2][0]
+    assert alone.sum() > 0
+    for k in range(5):
+        assert np.array_equal(irr[k], alone)
+    one.close()
+    b.close()

@@ -153,3 +153,17 @@ def test_unsupported_integrator_is_refused(cuda):
     with pytest.raises(_lib.OweHipError) as e:
         render.Renderer(S.white_furnace_scene(0.5), S.settings(integrator=7))
     assert e.value.code == _lib.ERR_UNSUPPORTED
+
+
+def test_the_first_image_takes_no_memory(cuda):
+    import torch
+
+    r = render.Renderer(S.dispersion_prism_scene(1024, 1024), S.settings(seed=1, max_depth=4))
+    r.set_mode(render.Renderer.PERSISTENT)
+    r.run_pass(1)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    image = r.resolve()
+    assert torch.cuda.mem_get_info()[0] == free
+    assert np.isfinite(image).all() and image.sum() > 0
+    r.close()
