@@ -51,8 +51,8 @@ void launchParticlesRefill(bool contacts, const DScene* sc, const Settings& set,
 // ones. `left` is what the asking lane knew at its own last fetch, so it costs no load. Ids stay a partition
 // of the pass whatever the grain, and the films are integers, so images do not depend on it. With chunks of 4
 // on 768 blocks: pool at 256x192x16 5.3 -> 4.0 ms, a telescope's room at 251x203x16
-// 6.0 -> 3.8, prism at 256x256x64 1.50 -> 1.45, light tracing 0.54 -> 0.51. Half a share gives 4.1, 3.9, 1.55 and
-// 0.51, a whole share 4.6, 5.9, 1.49 and 0.54; chunks of 1 throughout 4.1, 3.8, 1.62 and 0.51.
+// 6.0 -> 3.8, light tracing 0.54 -> 0.51. Half a share gives 4.1, 3.9 and 0.51, a whole share 4.6, 5.9 and 0.54;
+// chunks of 1 throughout 4.1, 3.8 and 0.51.
 __device__ __forceinline__ uint32_t grainOf(uint64_t left, uint32_t chunk, uint32_t lanes) {
     return uint32_t(fmaxf(1.0f, fminf(float(chunk), float(left) / (4.0f * float(lanes)))));
 }

@@ -899,8 +899,14 @@ __global__ __launch_bounds__(kBlock, 2) void drainKernel(DScene sc, Settings set
 // lane in registers and advances it one segment per iteration (intersect, shade, shadow — the very
 // device functions of the wavefront kernels, so every path's float operations are the same); a lane
 // whose path ends splats it and takes the next path id from its chunk, or a new chunk of up to `chunk`
-// consecutive ids (grainOf) from a device counter (one atomic per wave per refill). Splats of consecutive
+// consecutive ids from a device counter (one atomic per wave per refill). Splats of consecutive
 // paths of one pixel accumulate in the lane and reach the film as one 64-bit atomic per channel.
+// A pass of fewer than four chunks a lane shrinks them toward its end (grainOf); a longer one keeps them whole, as the wait
+// at its end is a small part of it while smaller chunks cost each path its own adds to the film, which paths
+// of few segments do not hide. Whole / shrinking chunks of 4, 3 blocks a compute unit unless stated, ms: below the line
+// prism at 256x256x16 1.17 / 0.55, x32 1.23 / 0.83, lifted prism x32 1.02 / 0.75, room x32 11.8 / 9.0; above it lifted
+// prism x64 1.21 / 1.26 (4 blocks 1.23 / 1.30), x128 2.22 / 2.32, prism x64 on 2 blocks 1.48 / 1.54, x128 2.57 / 2.66,
+// and, the other way, room x64 21.4 / 18.7, dispersion_prism x64 3.31 / 2.75.
 // The film is integer, so it equals the wavefront's bit for bit.
 struct Persist {
     uint64_t total;            // paths of the pass: path g is sample g % spp of pixel g / spp
@@ -970,7 +976,8 @@ __device__ __forceinline__ uint32_t persistDrain(const DScene& sc, const Setting
             unsigned long long base = 0;
             uint32_t grain = 0;
             if (int(lane) == leader) {
-                grain = grainOf(a.total - end, a.chunk, gridDim.x * kBlock);
+                const uint32_t lanes = gridDim.x * kBlock;
+                grain = a.total < 4ull * a.chunk * lanes ? grainOf(a.total - end, a.chunk, lanes) : a.chunk;
                 base = atomicAdd(a.next, (unsigned long long)__popcll(ask) * grain);
             }
             base = __shfl(base, leader);

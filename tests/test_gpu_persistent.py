@@ -110,10 +110,12 @@ def test_autotune_picks_a_shape_and_leaves_no_trace(cuda):
     assert np.array_equal(w.resolve(), ref)
 
 
-@pytest.mark.parametrize("width,height,spp,chunk,blocks", [(101, 67, 170, 1024, 1), (64, 64, 16, 1024, 8), (3, 1, 1, 4, 2)])
+@pytest.mark.parametrize("width,height,spp,chunk,blocks", [(101, 67, 170, 1024, 1), (64, 64, 16, 1024, 8), (3, 1, 1, 4, 2),
+                                                           (512, 512, 2, 2, 1), (511, 513, 2, 2, 1)])
 def test_shrinking_chunks_trace_every_path_once(cuda, width, height, spp, chunk, blocks):
     # Chunks from a quarter of a lane's share down to one id: more ids than lanes by an odd factor, about one
-    # id a lane, and fewer ids than one wave's lanes. The film and the statistics are integers: no tolerance.
+    # id a lane, and fewer ids than one wave's lanes; at four chunks a lane, where they stay whole (256 compute units of
+    # 256 lanes), and two ids below. The film and the statistics are integers: no tolerance.
     sc = S.dispersion_prism_scene(width, height)
     st = S.settings(seed=12, **PRISM)
     a, sa = render_with(sc, st, spp, 2, False)
