@@ -681,10 +681,8 @@ __global__ __launch_bounds__(kPBlock) void particleKernel(DScene sc, Settings se
 // ends. Particle ids come in chunks of up to `chunk` (grainOf) from one device counter (one atomic per wave per
 // refill). The bins are integers, so the image equals particleKernel's bit for bit.
 template <bool kContacts>
-__global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene* __restrict__ scene, Settings set, ParticleBatch pb) {
-    const DScene& sc = *scene;
-    __shared__ uint32_t stack[kRefillStack * kPBlock];
-    PCtx c{sc, set, pb, stack + threadIdx.x};
+__device__ __forceinline__ void particleRefill(const DScene& sc, const Settings& set, const ParticleBatch& pb, uint32_t* stack) {
+    PCtx c{sc, set, pb, stack};
     c.sum[0] = c.sum[1] = c.sum[2] = 0.0f;
     c.segments = c.inconsistencies = c.leaks = 0;
     const bool observer = sc.obs.kind == OWE_DETECTOR_OBSERVER && !(set.mode & kModePartition);  // emitter seen directly
@@ -732,6 +730,20 @@ __global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene*
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             if (n[k]) atomicAdd(&pb.stats[k], (unsigned long long)n[k]);
+}
+
+// Two waves per SIMD, the scene's record read from memory: as an argument its hundred words are all loaded at the
+// start and spilled to vector lanes, 353 to 425 of them here.
+template <bool kContacts>
+__global__ __launch_bounds__(kPBlock, 2) void particleRefillKernel(const DScene* __restrict__ scene, Settings set, ParticleBatch pb) {
+    __shared__ uint32_t stack[kRefillStack * kPBlock];
+    particleRefill<kContacts>(*scene, set, pb, stack + threadIdx.x);
+}
+// One wave per SIMD with all of its registers, for grids that fill no more (launchParticlesRefill).
+template <bool kContacts>
+__global__ __launch_bounds__(kPBlock) void particleRefillWideKernel(DScene sc, Settings set, ParticleBatch pb) {
+    __shared__ uint32_t stack[kRefillStack * kPBlock];
+    particleRefill<kContacts>(sc, set, pb, stack + threadIdx.x);
 }
 
 // ---------------------------------------------------------------- vertex connection and merging
@@ -1005,12 +1017,18 @@ void launchVcmLight(bool contacts, const DScene* sc, const Settings& set, const 
     OWE_HIP_CHECK(hipGetLastError());
 }
 
-void launchParticlesRefill(bool contacts, const DScene* sc, const Settings& set, const ParticleBatch& b, uint32_t blocks,
-                           hipStream_t stream) {
+void launchParticlesRefill(const DScene& sc, const DScene* scene, const Settings& set, const ParticleBatch& b,
+                           uint32_t computeUnits, uint32_t blocksPerCU, hipStream_t stream) {
     if (b.total == 0) return;
-    const dim3 grid{std::max(1u, blocks)}, block{kPBlock};
-    if (contacts) hipLaunchKernelGGL((particleRefillKernel<true>), grid, block, 0, stream, sc, set, b);
-    else hipLaunchKernelGGL((particleRefillKernel<false>), grid, block, 0, stream, sc, set, b);
+    const dim3 grid{std::max(1u, computeUnits * blocksPerCU)}, block{kPBlock};
+    auto go = [&](auto kernel, auto record) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, record, set, b); };
+    if (blocksPerCU * (kPBlock / 64) <= 4) {  // four SIMDs to a compute unit
+        if (sc.contacts) go(particleRefillWideKernel<true>, sc);
+        else go(particleRefillWideKernel<false>, sc);
+    } else {
+        if (sc.contacts) go(particleRefillKernel<true>, scene);
+        else go(particleRefillKernel<false>, scene);
+    }
     OWE_HIP_CHECK(hipGetLastError());
 }
 

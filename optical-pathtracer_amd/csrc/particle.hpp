@@ -36,14 +36,15 @@ struct ParticleBatch {
 // traversal stack.
 void launchParticles(const DScene& sc, const Settings& set, const ParticleBatch& b, uint32_t stackCap,
                      hipStream_t stream);
-// Enqueues the pass in the lane-refill form on a grid of `blocks` blocks (the scene's stack bound
-// must not exceed 48). sc: the scene's record in device memory. As a kernel argument its hundred
-// words are all loaded at the start and spilled to vector lanes, 353 to 425 of them in this kernel: read from memory
-// instead, and held to two waves per SIMD where it took the registers of one, the prism's 1,048,576 particles
-// with reset and resolve go from 0.80 to 0.70 ms and 16 vcm iterations at 256² from 3.24 to 3.11 ms. (The camera
-// paths' persistent kernel is 3 to 5 % faster with the argument.)
-void launchParticlesRefill(bool contacts, const DScene* sc, const Settings& set, const ParticleBatch& b, uint32_t blocks,
-                           hipStream_t stream);
+// Enqueues the pass in the lane-refill form on a grid of `blocksPerCU` blocks to each compute unit (the scene's stack
+// bound must not exceed 48). scene: sc in device memory. Grids of more than one wave to a SIMD run the kernel held to two,
+// which reads the record from memory (the prism's 1,048,576 particles with reset and resolve 0.80 -> 0.70 ms, 16
+// vcm iterations at 256² 3.24 -> 3.11; 8,388,608 particles on 4 blocks 3.40 -> 2.30). Smaller grids run the one that
+// takes it as an argument and all registers: on 2 and 1 blocks the other one takes 3.66 and 6.67 ms there, this one
+// 3.40 and 6.26 (lifted prism 3.28 / 3.22, 5.98 / 5.81). (The camera paths' persistent kernel is 3 to 5 % faster with the
+// argument.)
+void launchParticlesRefill(const DScene& sc, const DScene* scene, const Settings& set, const ParticleBatch& b,
+                           uint32_t computeUnits, uint32_t blocksPerCU, hipStream_t stream);
 
 // How many consecutive ids a lane of the refilling kernels takes when at most `left` are left to a grid of
 // `lanes` lanes: `chunk`, but no more than a quarter of a lane's even share. A lane traces its ids one after

@@ -2250,7 +2250,7 @@ void runParticles(owe_hip_renderer* r, uint64_t total, uint32_t pass, const uint
         b.regen = r->regen;
         OWE_HIP_CHECK(hipMemsetAsync(r->particleNext, 0, sizeof(unsigned long long), r->stream));
         timed(r, kShade, [&] {
-            launchParticlesRefill(r->dev.contacts != 0u, r->scene, r->set, b, uint32_t(std::max(1, r->computeUnits * r->blocksPerCU)), r->stream);
+            launchParticlesRefill(r->dev, r->scene, r->set, b, uint32_t(r->computeUnits), uint32_t(r->blocksPerCU), r->stream);
         });
     } else {
         // One thread per particle, in launches of at most `capacity` particles.
