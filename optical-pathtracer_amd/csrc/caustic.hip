@@ -1,6 +1,6 @@
 // Differentiable caustic design: owe_hip_caustic_* of include/owe_hip_caustic.h.
 //
-// Forward: one thread per particle, each wave over a contiguous range of particles. A particle of
+// Forward: one thread per particle, each block over a contiguous range of particles. A particle of
 // pass k is stream (hashCombine(seed, i), k): a wavelength importance-sampled over the visible range
 // and weighted by the sun's luminous spectrum, and a point on the slab's entry face, stratified over
 // square tiles (a wave's particles share a tile or two). It enters at normal incidence (weight 1 − R),
@@ -11,9 +11,9 @@
 // reproducible.
 //
 // Backward (path replay): the same particles are drawn again from their seeds and the same float
-// operations give the same wall point; the exit computation is also carried through three-component
-// dual numbers (∂/∂h, ∂/∂h_x, ∂/∂h_y at the particle's exit point), which with the spline weights
-// and ∂L/∂E at the nine pixels gives ∂L/∂(h, h_x, h_y) for this particle. h, h_x and h_y are linear in
+// operations give the same wall point; the exit's derivatives (by h, h_x and h_y at the particle's exit
+// point, exitSlopes) with the spline weights
+// and ∂L/∂E at the nine pixels give ∂L/∂(h, h_x, h_y) for this particle. h, h_x and h_y are linear in
 // the 4 × 4 heights around the cell (bicubic Hermite patch with central-difference node slopes), so
 // the particle adds its share to those sixteen heights: no stored paths. Both passes gather their
 // adds (pixels, nodes) in the block's table in LDS and send each touched pixel or node to HBM once
@@ -46,8 +46,8 @@ constexpr double kSplatUnits = 4294967296.0;  // fixed-point units per unit of i
 struct CArgs {
     const float* heights;
     uint32_t nodes, pixels;
-    float slabHalf, cell, z0, zWall, wallHalf, pix;
-    float perCell, perPix;   // 1 / cell, 1 / pix
+    float slabHalf, z0, zWall, wallHalf;
+    float perCell, perPix;   // cells and pixels to a metre
     uint64_t particles, seed, pass;
     DMedium slab, air;
     // The sun's B(λ) / ∫ B ȳ = sunScale e / (λ⁵ (1 − e sunRef)) with e = exp(sunAt − sunC2 / λ), λ in µm: the exponent is
@@ -530,11 +530,9 @@ CArgs makeArgs(const owe_caustic_settings& s) {
     a.nodes = s.nodes;
     a.pixels = s.pixels;
     a.slabHalf = float(s.slab_half);
-    a.cell = float(2 * s.slab_half / (s.nodes - 1));
     a.z0 = float(s.thickness);
     a.zWall = float(s.wall_z);
     a.wallHalf = float(s.wall_half);
-    a.pix = float(2 * s.wall_half / s.pixels);
     a.perCell = float((s.nodes - 1) / (2 * s.slab_half));
     a.perPix = float(s.pixels / (2 * s.wall_half));
     a.particles = s.particles;

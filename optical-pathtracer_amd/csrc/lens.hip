@@ -11,12 +11,12 @@
 // different ray counts (4k to 1M) share the launch without tails of idle blocks.
 //
 // Ray–surface roots follow SagSurface (src/owe/scene/geometry.cpp:115-166,
-// src/owe/core/shared/surfaces.hpp:13-94) in float32 with the reference's float tolerances; each
-// quadric root is then re-solved from the approximate hit point (refineRoot) — in float64 on a
-// steep surface (|c|·r_max > 0.5), where the quadric's terms cancel, and throughout instruments with
-// mirrors or without focal power (metre paths, high angular magnification), in float elsewhere — and a
-// numeric asphere root is polished by Newton steps in float64: the only fp64 of the per-ray path
-// (the spot sums are accumulated in double from float per-ray terms). Transmission is the walk's
+// src/owe/core/shared/surfaces.hpp:13-94) with the reference's float tolerances. A conic or flat row is met from
+// its vertex plane by the small root (conicHit): in float64 on a steep surface (|c|·r_max > 0.5) and
+// throughout instruments with mirrors or without focal power (metre paths, high angular magnification), in
+// float32 elsewhere. Where another root may come first, and on aspheres, sagHit decides: a float quadric root
+// re-solved from the approximate hit point, a numeric asphere root polished by Newton steps in float64. Gaps
+// between rows are subtracted in double and the spot sums accumulated in double. Transmission is the walk's
 // deterministic refraction with weight T = 1 − R (transport.cpp:531-595); TIR or a missed aperture
 // ends a ray.
 #include <hip/hip_runtime.h>

@@ -372,3 +372,63 @@ def test_results_take_no_memory_and_pieces_of_the_grids_join(cuda):
         assert np.array_equal(irr[k], alone)
     one.close()
     b.close()
+
+
+@pytest.mark.parametrize("planes,pixels,step", [(16, 1024, 2e-3), (2, 4096, 50e-3)])
+def test_grids_of_many_more_bins_than_the_table(cuda, planes, pixels, step):
+    """Defocused light over 50,000 bins and more of a lens, where a block's table holds 4,096: every add that finds no place goes
+    to memory. The bins are those of the traced rays, but for rays within float rounding of an edge (a pixel
+    is 24 µm or 6, a coordinate on the plane rounds to 5 nm: below 1 in 1,000), and no launch shape changes them."""
+    p = L.Prescription(L.SINGLET.surfaces, rays=150_000)
+    half = 12.5e-3
+    st = L.c_settings(wavelengths=(587.56,), half_size=half, pixels=pixels, planes=planes, focus_step=step)
+    b = L.LensBatch([p], st)
+    grids = []
+    for shape in ((3, 1024), (1, 256), (2, 16384)):
+        b.set_shape(*shape)
+        b.run()
+        per, _, irr = b.results(irradiance=True)
+        grids.append(irr[0].astype(np.float64))
+    assert np.array_equal(grids[0], grids[1]) and np.array_equal(grids[0], grids[2])
+    r = b.trace(0, 0, np.arange(p.rays, dtype=np.uint64))
+    b.close()
+    r = r[r[:, 6] > 0]
+    z0 = per[0]["last_vertex_z"] + per[0]["bfl"]
+    y0 = per[0]["efl"] * math.tan(math.radians(st.field_deg))
+    beam = math.pi * (0.999 * per[0]["entrance_pupil_radius"]) ** 2 * math.cos(math.radians(st.field_deg))
+    unit = beam / (p.rays * (2 * half / pixels) ** 2)
+    moved = touched = 0.0
+    for k in range(planes):
+        s = (z0 + (k - 0.5 * (planes - 1)) * step - r[:, 2]) / r[:, 5]
+        x = ((r[:, 0] + r[:, 3] * s) / half + 1) * 0.5 * pixels
+        y = (1 - (r[:, 1] + r[:, 4] * s - y0) / half) * 0.5 * pixels
+        ok = (x >= 0) & (y >= 0) & (x < pixels) & (y < pixels)
+        want = np.bincount((y[ok].astype(int) * pixels + x[ok].astype(int)), r[ok, 6], pixels * pixels) * unit
+        touched += (want > 0).sum()
+        moved += np.abs(grids[0][k].ravel() - want).sum() / want.sum() / 2
+    print(f"{planes} planes of {pixels}²: {int(touched)} bins, {moved / planes:.2e} of the light in another bin", flush=True)
+    assert touched > 50_000 and moved / planes < 1e-3
+
+
+def test_mirrors_behind_many_rows_obstruct(cuda, oracle):
+    """33 thin plates before a Gregorian: its mirrors are rows 66 and 67, beyond the first 64, and the secondary (21 mm of 54) stops
+    the centre of the beam on its way to the primary, 15 % where the primary's bore alone takes 6. Point and direction as for the telescope by itself: 24 µm of
+    glass and 0.9 m of travel, coordinates of 5 cm that round to 4e-9 m, angles magnified 54 times."""
+    tele = L.solve_afocal(L.GREGORIAN, 587.5618)
+    rows = []
+    for _ in range(33):
+        rows += [L.Surface(math.inf, 0.01, "N-BK7", 60.0), L.Surface(math.inf, 0.01, "air", 60.0)]
+    rows[-1].t = 700.0
+    p = L.Prescription(rows + tele.surfaces, rays=8192)
+    b = L.LensBatch([p], L.c_settings(field_deg=0.05, pixels=0, reference=587.5618))
+    lo = LensOracle(oracle, [p], field_deg=0.05, reference=587.5618)
+    idx = np.arange(8192, dtype=np.uint64)
+    g, c = b.trace(0, 4, idx), lo.trace(0, L.FRAUNHOFER7[4], idx)
+    b.close()
+    assert [k for k, s in enumerate(p.surfaces) if s.reflect] == [66, 67]
+    okg, okc = g[:, 6] > 0, c[:, 6] > 0
+    both = okg & okc
+    dp, dd = np.abs(g[both, :3] - c[both, :3]).max(), np.abs(g[both, 3:6] - c[both, 3:6]).max()
+    print(f"{both.sum()} of {len(idx)} arrive on both, {(okg != okc).sum()} flips, |Δp| {dp:.1e}, |Δd| {dd:.1e}", flush=True)
+    assert 1000 < both.sum() < 8192 * 0.9 and (okg != okc).sum() <= 4
+    assert dp < 1e-7 and dd < 1e-5
