@@ -1137,12 +1137,13 @@ int owe_hip_lens_batch_autotune(owe_hip_lens_batch* b, double* best_ms) {
             layoutItems(b, c.rays);
             return runOnce(b);
         };
-        // Up to the resident blocks (48 achromats with three, four and eight 1.023, 1.016 and 1.018 ms; six small lenses with
-        // two, four and eight 0.021, 0.027 and 0.037), and the batch's own item.
+        // Up to the resident blocks, and grids of more, whose chunks are smaller (chunkOf): 256 achromats take 15.1 ms
+        // with eight blocks and 19.1 with three, 48 achromats 1.02 with three, four and eight, six small lenses 0.021 with
+        // two and 0.037 with eight. And the batch's own item.
         std::vector<uint32_t> items{256u, 1024u, 4096u, 16384u};
         const uint32_t own = defaultItem(b);
         if (std::find(items.begin(), items.end(), own) == items.end()) items.push_back(own);
-        for (int blocks = 1; blocks <= kResidentBlocks; ++blocks)
+        for (int blocks : {1, 2, kResidentBlocks, 4, 8})
             for (uint32_t rays : items) {
                 cands.push_back({blocks, rays, 0.0});
                 cands.back().ms = run(cands.back());
