@@ -177,7 +177,8 @@ int owe_hip_renderer_particles(owe_hip_renderer* renderer, int pass, const uint6
  * the default) and the persistent batched form (a grid sized to the chip drains a device queue of
  * path ids, each lane tracing a path to its end in registers with the same device functions). The
  * film is integer, so both give the same image bit for bit. blocks_per_cu and chunk (path ids per
- * lane fetch) shape the persistent launch (0 keeps the current value); waves_per_simd (2 or 3; 0
+ * lane fetch; fewer toward the end of a pass of fewer than four chunks a lane) shape the persistent
+ * launch (0 keeps the current value); waves_per_simd (2 or 3; 0
  * keeps it) selects the persistent kernel compiled for that many resident waves per SIMD (3 trades
  * register spills for latency hiding); refill (1..64; 0 keeps it) is how many of a wave's lanes must
  * have finished their paths before the wave starts new ones together; use_graph replays each pass
@@ -185,7 +186,7 @@ int owe_hip_renderer_particles(owe_hip_renderer* renderer, int pass, const uint6
  * A light-integrator renderer has the same two modes for its particle pass: one thread per particle
  * (OWE_HIP_MODE_WAVEFRONT, the reference's particle kernel's form, the default) or the lane-refill
  * form (OWE_HIP_MODE_PERSISTENT: a grid of blocks_per_cu blocks per compute unit, each lane advancing
- * its particle a segment at a time and taking chunk particle ids at a time, refill as above;
+ * its particle a segment at a time and taking up to chunk particle ids at a time, refill as above;
  * waves_per_simd and use_graph do not apply). Both give the same image bit for bit. */
 #define OWE_HIP_MODE_WAVEFRONT 0
 #define OWE_HIP_MODE_PERSISTENT 1
@@ -212,7 +213,7 @@ int owe_hip_renderer_get_vcm_in_flight(const owe_hip_renderer* renderer, int* it
 int owe_hip_renderer_autotune(owe_hip_renderer* renderer, int spp, double* best_ms);
 
 /* The autotuner's per-device tuning cache: a text file of tuned shapes, one line per (device,
- * form, pass size, flattened scene, settings) key. owe_hip_renderer_autotune first looks its key
+ * form, pass size, flattened scene, settings, generation of the kernels) key. owe_hip_renderer_autotune first looks its key
  * up there (a hit applies the recorded shape without sweeping and reports its recorded time) and
  * appends what a sweep chooses. path NULL or "" disables it; the default is the environment
  * variable OWE_HIP_TUNING_CACHE, else none. Process-wide. */

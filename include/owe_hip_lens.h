@@ -133,8 +133,9 @@ int owe_hip_lens_batch_run(owe_hip_lens_batch* batch);
  * (n_lenses × focus_planes × pixels × pixels floats, unit incident irradiance across the beam,
  * plane 0 nearest the lens; may be null). */
 int owe_hip_lens_batch_results(owe_hip_lens_batch* batch, owe_lens_result* lenses, double* moments, float* irradiance);
-/* The persistent launch's shape: resident blocks per compute unit and rays per work item (a
- * multiple of 64); 0 keeps the current value. */
+/* The persistent launch's shape: blocks per compute unit in the grid and rays per work item (a
+ * multiple of 64; an item takes the next whole number of rays to each of a block's 256 threads); 0 keeps the
+ * current value. */
 int owe_hip_lens_batch_set_shape(owe_hip_lens_batch* batch, int blocks_per_cu, int rays_per_item);
 /* Times runs under candidate shapes, keeps the fastest; best_ms (optional) receives its time. */
 int owe_hip_lens_batch_autotune(owe_hip_lens_batch* batch, double* best_ms);

@@ -8,11 +8,11 @@
 // rays to a wave. Per step a wave either visits a node or tests triangles, two a lane at most, in all the lanes that are
 // at one (traverse.hpp): a ray meets a leaf in one node of eight, so testing the leaves of a node where
 // it is visited, as the transport kernels' traverseBvh4 does, ran the triangle test with 1 to 5 lanes
-// of 64. Bound by the bytes beyond L2 (85 M lines of 128 bytes for 8,388,608 closest queries on
-// 1,048,820 triangles, 90 MB of nodes and triangles against 4 MiB of L2 per XCD), no longer by VALU
-// issue: 4.02 → 1.89 ms closest and 3.05 → 1.51 ms any hit; 0.48 → 0.29 and 0.35 → 0.19 ms for 1,000,003
-// rays on 100,820 triangles; 4,096 rays on 20,480 triangles, bound by the longest ray's chain of
-// loads, stay at 0.033 and go from 0.028 to 0.025 ms.
+// of 64. Near two limits at once: 10.2 GB beyond L2 for 8,388,608 closest queries on 1,048,820 triangles (90 MB of
+// nodes and triangles against 4 MiB of L2 per XCD) at the rate of a large copy, and VALU busy 91 % of the time with half
+// of the lanes. Launches back to back: 4.02 → 1.90 ms closest and 3.05 → 1.46 ms any hit; 0.48 → 0.27 and
+// 0.35 → 0.19 ms for 1,000,003 rays on 100,820 triangles. 4,096 rays on 20,480 triangles take 33 µs closest and 28 any
+// hit, as before: the longest ray's chain of loads (the host's call is 7 µs, and waiting for it adds 15).
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -47,7 +47,7 @@ constexpr int kQueryBlock = 128;
 // at once; lanes end out of order, so the lines fill in a few partial writes that L2 gathers.
 // The triangle step runs when the lanes at a leaf are half as many as those at a node, or when none is at
 // a node: of thresholds from a quarter to one and a half, and of fixed counts from 1 to 32, this one
-// was the fastest closest query (2.01 ms with one triangle a step; 8 lanes fixed 2.4, 24 lanes fixed 2.3) and none was faster for any hit.
+// was the fastest closest query (2.0 ms with one triangle a step; 8 lanes fixed 2.4, 24 lanes fixed 2.3) and none was faster for any hit.
 template <bool kAny>
 __global__ __launch_bounds__(kQueryBlock) void traceKernel(const WideNode* __restrict__ nodes,
                                                            const TriRecord* __restrict__ tris,

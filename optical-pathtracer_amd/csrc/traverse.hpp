@@ -130,7 +130,7 @@ __device__ inline RayHit traverseBvh4(const WideNode* __restrict__ nodes, const 
 // order, and the top is entered next; what a ray visits, and in which order, depends on the ray
 // alone and not on its wave. Culling happens when a node is visited: keeping each entry's distance to
 // cull it when popped saves a fifth of a closest query's visits (13.4 of 16.6 on the 1,048,820-triangle
-// mesh) but its longer pops cost more than that (2.33 against 2.01 ms for 8,388,608 rays).
+// mesh) but its longer pops cost more than that (2.33 against 2.0 ms for 8,388,608 rays, one triangle a step).
 struct Walk {
     f3 o, d, inv;
     Shear sh;
@@ -256,8 +256,8 @@ __device__ __forceinline__ void walkNode(Walk& w, const WideNode* __restrict__ n
 
 // Tests the first two triangles of leaf reference w.cur (its only one where it has one) and moves to its next
 // ones, or to the stack's top. Both are loaded together: one wait for two tests, where one triangle a step
-// took 1.99 ms for 8,388,608 closest queries, 0.207 for 1,000,003 any-hit ones and 0.056 for 4,096 (with two 1.89, 0.199
-// and 0.053).
+// took 2.0 ms for 8,388,608 closest queries and 0.207 for 1,000,003 any-hit ones (with two 1.9 and 0.199; 4,096 queries
+// take the same with either).
 template <bool kAny>
 __device__ __forceinline__ void walkTriangle(Walk& w, const TriRecord* __restrict__ tris, const WalkStack& st,
                                              uint32_t stride) {
